@@ -33,7 +33,7 @@ KIND_NAMES = ["gemm64_rc_pre", "gemm64_rc_row", "gemm64_cr_pre", "gemm64_cc", "g
               "phase", "tcvt64to32", "diag64x32", "gemm64_cc_sub", "lu_shape", "block", "sigma", "gather",
               "tblock", "trsm", "gemm32_rc_pre_diag", "dreduce", "rgather", "gemm32_rc_diag", "tscale64to32",
               "gemm32_rck_diag", "colscale64to32", "lu_shape_defer",
-              "gemm64_cc4", "gemm64_cc4_sub"]
+              "gemm64_cc4", "gemm64_cc4_sub", "suffix64_chains", "right32_chains", "right64_chains"]
 
 
 def parse():
@@ -652,15 +652,15 @@ def main():
                 "force_ms": float(prof[:, 1].sum()),
                 "breakdown_ms": {KIND_NAMES[k]: round(float(prof[k, 1]), 4) for k in range(nk) if prof[k, 0] > 0}}
 
-    # the FP32 right-chain step, the chain kernel furthest below its peak, beside the dominant one
-    k32 = KIND_NAMES.index("gemm32_rck_diag")
+    # the FP32 right chains, the chain kernel furthest below its peak, beside the dominant one
+    k32 = KIND_NAMES.index("right32_chains")
     if prof[k32, 0] > 0:
         a32 = prof[k32, 2] / prof[k32, 1] * 1e3 / 1e12
-        roofline["fp32_right_chain"] = {"kernel": "gemm32_rck_diag", "achieved": a32, "peak": PEAK["f32"],
+        roofline["fp32_right_chain"] = {"kernel": "right32_chains", "achieved": a32, "peak": PEAK["f32"],
                                         "unit": "TFLOP/s", "frac": a32 / PEAK["f32"],
                                         "avg_launch_ms": float(prof[k32, 1] / prof[k32, 0]),
-                                        "note": "epilogue-bound: the force diagonal reads the FP64 suffix "
-                                                "entries (16 B per product element) after the K loop"}
+                                        "note": "whole right chains per launch; the force diagonal reads the FP64 "
+                                                "suffix entries (16 B per product element) beside the MFMAs"}
     progress("roofline done")
     # ---------------- plain FP64, one chain, unbatched (from chain 0's thermalised field)
     plain = None

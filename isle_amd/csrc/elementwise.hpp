@@ -156,15 +156,16 @@ __global__ __launch_bounds__(256) void diag_prod_kernel(const DiagItem<TL, TR>* 
     }
 }
 
-// out[i] (interleaved complex) = sum over s < slots of part[(s * n + i) * 2 + {0, 1}]: the
-// per-16-column partial row sums written by a FUSED_DIAG chain product.
+// out[off + i] (interleaved complex) = sum over s < slots of part[(s * n + i) * 2 + {0, 1}]: the
+// per-16-column partial row sums written by a FUSED_DIAG chain product or a right chain.
 struct DReduceItem {
     const double* part;
-    double* out;
+    long off;  // complex elements into out
     int n, slots;
 };
 
-__global__ __launch_bounds__(256) void diag_reduce_kernel(const DReduceItem* __restrict__ items) {
+__global__ __launch_bounds__(256) void diag_reduce_kernel(const DReduceItem* __restrict__ items,
+                                                          double* __restrict__ out) {
     const DReduceItem it = items[blockIdx.y];
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= it.n) return;
@@ -173,8 +174,8 @@ __global__ __launch_bounds__(256) void diag_reduce_kernel(const DReduceItem* __r
         sr += it.part[((long)s * it.n + i) * 2];
         si += it.part[((long)s * it.n + i) * 2 + 1];
     }
-    it.out[2 * i] = sr;
-    it.out[2 * i + 1] = si;
+    out[2 * (it.off + i)] = sr;
+    out[2 * (it.off + i) + 1] = si;
 }
 
 // ---------------------------------------------------------------------------

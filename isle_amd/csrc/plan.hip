@@ -14,6 +14,16 @@ namespace {
 
 constexpr int EW_THREADS = 256;
 
+// A group's K: re plane, im plane `plane` doubles after it, row stride ld, factor sign.
+struct ChainK {
+    const double* re;
+    long plane;
+    long ld;
+    double sign;
+};
+
+}  // namespace
+
 // Host-side staging of one cached operation.
 struct Builder {
     OpCache& op;
@@ -36,12 +46,23 @@ struct Builder {
         size_t off = (blob.size() + 63) & ~size_t(63);
         blob.resize(off + items.size() * sizeof(It));
         std::memcpy(blob.data() + off, items.data(), items.size() * sizeof(It));
-        pend.push_back({kind, off, (int)items.size(), mm, mn, flag, aux, flops_of(kind, items), tile, sizeof(It)});
+        pend.push_back({kind, off, (int)items.size(), mm, mn, flag, aux, flops_of(kind, items, mm), tile, sizeof(It)});
     }
     template <typename It>
-    static double flops_of(K, const std::vector<It>&) { return 0.0; }
+    static double flops_of(K, const std::vector<It>&, int) { return 0.0; }
+    static double flops_of(K, const std::vector<SuffixItem>& items, int n) {
+        double f = 0;
+        for (const auto& g : items) f += 4.0 * n * (double)n * n * (g.count - 1);
+        return f;
+    }
     template <typename T>
-    static double flops_of(K kind, const std::vector<GemmItem<T>>& items) {
+    static double flops_of(K, const std::vector<RightItem<T>>& items, int n) {
+        double f = 0;
+        for (const auto& g : items) f += 4.0 * n * (double)n * n * g.count;
+        return f;
+    }
+    template <typename T>
+    static double flops_of(K kind, const std::vector<GemmItem<T>>& items, int) {
         const double reals = (kind == K::GEMM64_CC || kind == K::GEMM64_CC_SUB || kind == K::TRSM ||
                               kind == K::GEMM64_CC4 || kind == K::GEMM64_CC4_SUB) ? 4.0 : 2.0;
         double f = 0;
@@ -69,6 +90,8 @@ struct Builder {
         op.blob = std::move(blob);
     }
 };
+
+namespace {
 
 // complex n x n matrix (split planes) inside a block array
 template <typename T>
@@ -205,6 +228,121 @@ void add_trsm(Builder& b, int mode, int n, int w, const std::vector<TrsmMat>& ma
         }
     }
 }
+// Top level of the grouped force in FP64, from the group products P(item, j):
+//   GL_{ng-1} = I, GL_j = P_{j+1} GL_{j+1};  Mid = (1 + P_0 GL_0)^{-1}
+//   RR_0 = Mid, RR_j = RR_{j-1} P_{j-1};     K_j = GL_j RR_j
+// trsm: the inverse by blocked triangular solves on GEMMs (n % 32 == 0; many matrices), else by
+// lu_solve_kernel (few: one launch instead of four per pair of panels).
+struct TopLevel {
+    double *KK, *RR;
+    int ng;
+    long nn;
+    const double* k(int item, int j) const {  // K_j: re plane, im plane nn after it
+        return (j < ng - 1 ? KK : RR) + ((long)item * ng + j) * 2 * nn;
+    }
+};
+template <typename PF>
+TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm) {
+    const long nn = (long)n * n;
+    double* GL = b.d64((size_t)nb * ng * 2 * nn);
+    double* RR = b.d64((size_t)nb * ng * 2 * nn);
+    double* KK = b.d64((size_t)nb * ng * 2 * nn);
+    double* LUb = b.d64((size_t)nb * 2 * nn);
+    int* piv = b.di((size_t)nb * n);
+    auto m64 = [&](double* base, int item, int j) { return cmat(base, (long)item * ng + j, nn); };
+    if (ng == 1) {
+        std::vector<CopyItem<double, double>> cp;
+        for (int item = 0; item < nb; ++item) cp.push_back({mP(item, 0).re, LUb + (long)item * 2 * nn, 2 * nn});
+        b.add(K::COPY64, cp, (int)(2 * nn));
+    } else {
+        std::vector<CopyItem<double, double>> cp;
+        for (int item = 0; item < nb; ++item) cp.push_back({mP(item, ng - 1).re, m64(GL, item, ng - 2).re, 2 * nn});
+        b.add(K::COPY64, cp, (int)(2 * nn));
+        for (int j = ng - 3; j >= 0; --j) {
+            std::vector<GemmItem<double>> gi;
+            for (int item = 0; item < nb; ++item) {
+                const CMat<double> a = mP(item, j + 1), bb = m64(GL, item, j + 1);
+                gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(GL, item, j), nullptr, nullptr, nullptr,
+                                           nullptr, n));
+            }
+            b.add(K::GEMM64_CC, gi, n, n);
+        }
+        std::vector<GemmItem<double>> gi;
+        for (int item = 0; item < nb; ++item) {
+            const CMat<double> a = mP(item, 0), bb = m64(GL, item, 0);
+            gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, cmat(LUb, item, nn), nullptr, nullptr, nullptr,
+                                       nullptr, n));
+        }
+        b.add(K::GEMM64_CC, gi, n, n);
+    }
+    {
+        std::vector<LuItem> lu;
+        double* luw = b.d64(nb * lu_work_doubles(n));
+        for (int item = 0; item < nb; ++item)
+            lu.push_back({LUb + (long)item * 2 * nn, LUb + (long)item * 2 * nn + nn, piv + (long)item * n, nullptr,
+                          luw + item * lu_work_doubles(n), n, n});
+        b.add(K::LU, lu, n, 0, 1);
+        if (trsm) {
+            // Mid = (1 + P_0 GL_0)^{-1} = U^{-1} L^{-1} P: the row-permuted identity, then two
+            // blocked triangular solves on GEMMs
+            int* sig = b.di((size_t)nb * n);
+            double* S1 = b.d64((size_t)nb * 2 * nn);
+            double* S2 = b.d64((size_t)nb * 2 * nn);
+            std::vector<SigmaItem> sv;
+            std::vector<GatherItem> ga;
+            std::vector<TrsmMat> tl, tu;
+            for (int item = 0; item < nb; ++item) {
+                const CMat<double> s1 = cmat(S1, item, nn), s2 = cmat(S2, item, nn), rr = m64(RR, item, 0);
+                const double* fre = LUb + (long)item * 2 * nn;
+                sv.push_back({piv + (long)item * n, sig + (long)item * n, n, n});
+                ga.push_back({sig + (long)item * n, nullptr, nullptr, s1.re, s1.im, nullptr, nullptr, n, n, n, n, 0});
+                tl.push_back({fre, fre + nn, n, luw + item * lu_work_doubles(n), s1.re, s1.im, n, s2.re, s2.im, n});
+                tu.push_back({fre, fre + nn, n, luw + item * lu_work_doubles(n), s2.re, s2.im, n, rr.re, rr.im, n});
+            }
+            b.add(K::SIGMA, sv);
+            b.add(K::GATHER, ga, n, 0, 0, n);
+            add_trsm(b, 0, n, n, tl);
+            add_trsm(b, 1, n, n, tu);
+        } else {
+            std::vector<SolveItem> sv;
+            for (int item = 0; item < nb; ++item) {
+                SolveItem si{};
+                si.lu_re = LUb + (long)item * 2 * nn;
+                si.lu_im = si.lu_re + nn;
+                si.piv = piv + (long)item * n;
+                si.dinv = luw + item * lu_work_doubles(n);
+                si.x_re = m64(RR, item, 0).re;
+                si.x_im = m64(RR, item, 0).im;
+                si.xsr = n;
+                si.xsc = 1;
+                si.n = n;
+                si.ld = n;
+                si.nrhs = n;
+                sv.push_back(si);
+            }
+            b.add(K::SOLVE, sv, n, n);
+        }
+    }
+    for (int j = 1; j < ng; ++j) {
+        std::vector<GemmItem<double>> gi;
+        for (int item = 0; item < nb; ++item) {
+            const CMat<double> a = m64(RR, item, j - 1), bb = mP(item, j - 1);
+            gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(RR, item, j), nullptr, nullptr, nullptr, nullptr, n));
+        }
+        b.add(K::GEMM64_CC, gi, n, n);
+    }
+    if (ng > 1) {
+        std::vector<GemmItem<double>> gi;
+        for (int item = 0; item < nb; ++item)
+            for (int j = 0; j < ng - 1; ++j) {
+                const CMat<double> a = m64(GL, item, j), bb = m64(RR, item, j);
+                gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(KK, item, j), nullptr, nullptr, nullptr,
+                                           nullptr, n));
+            }
+        b.add(K::GEMM64_CC, gi, n, n);
+    }
+    return {KK, RR, ng, nn};
+}
 }  // namespace
 
 Plan::Plan(int hopping, int nx, const double* kappa, double mu, int sk)
@@ -259,6 +397,23 @@ Plan::Plan(int hopping, int nx, const double* kappa, double mu, int sk)
     for (int s = 0; s < 2; ++s) {
         hipLaunchKernelGGL((convert_kernel<double, float>), dim3(ew_blocks(nn)), dim3(EW_THREADS), 0, nullptr,
                            a64_[s]->as<double>(), a32_[s]->as<float>(), (long)nn);
+        ISLE_HIP(hipGetLastError());
+        if (!chain_fits(n)) continue;
+        const long e64 = (long)chain_packed_elems<double>(n), e32 = (long)chain_packed_elems<float>(n);
+        pk64_[s].reset(new DevBuf(e64 * sizeof(double)));
+        pk32_[s].reset(new DevBuf(e32 * sizeof(float)));
+        hipLaunchKernelGGL(chain_pack_kernel<double>, dim3(ew_blocks(e64)), dim3(256), 0, nullptr, a64_[s]->as<double>(),
+                           n, pk64_[s]->as<double>(), e64);
+        ISLE_HIP(hipGetLastError());
+        hipLaunchKernelGGL(chain_pack_kernel<float>, dim3(ew_blocks(e32)), dim3(256), 0, nullptr, a64_[s]->as<double>(),
+                           n, pk32_[s]->as<float>(), e32);
+        ISLE_HIP(hipGetLastError());
+    }
+    if (hop_ == EXP && chain_fits(n)) {
+        const long e64 = (long)chain_packed_elems<double>(n);
+        pke64_.reset(new DevBuf(e64 * sizeof(double)));
+        hipLaunchKernelGGL(chain_pack_kernel<double>, dim3(ew_blocks(e64)), dim3(256), 0, nullptr,
+                           e64_[PARTICLE]->as<double>(), n, pke64_->as<double>(), e64);
         ISLE_HIP(hipGetLastError());
     }
     ISLE_HIP(hipDeviceSynchronize());
@@ -320,10 +475,61 @@ void Plan::slice_matrix(int species, int inv, double* out_host) {
     ISLE_HIP(hipMemcpy(out_host, src.p, nn * 8, hipMemcpyDeviceToHost));
 }
 
+// Suffix chains of all groups of all (field, species) items in one launch: S_e at out(item, j),
+// the next ones `step` doubles further each (all = 1), or only S_s (all = 0).
+template <typename OF>
+void Plan::add_suffix(Builder& b, int nt, int g, int nb, int nspecies, const double* ph, OF out, long step, int all) {
+    const int n = nx_;
+    std::vector<SuffixItem> v;
+    for (int item = 0; item < nb; ++item)
+        for (int j = 0; j < nt / g; ++j) {
+            const double* d = ph + (long)item * 2 * nt * n;
+            const int s = item % nspecies;
+            v.push_back({pk64_[s]->as<double>(), a64_[s]->as<double>(), d, d + (long)nt * n, out(item, j), step,
+                         j * g + g - 1, -1, g, all, 0});
+        }
+    b.add(K::SUFFIX64, v, n, n);
+}
+
+// Right chains of all groups in one launch (FP32 with ph32, else FP64), their force diagonal summed
+// over the strips into the parts; Suf: nt matrices per item.
+template <typename KF>
+void Plan::add_right(Builder& b, OpCache& op, int nt, int g, int nb, int nspecies, const double* ph,
+                     const float* ph32, const double* Suf, KF kf) {
+    const int n = nx_, slots = chain_tiles(n);
+    const long nn = (long)n * n;
+    double* part = b.d64((size_t)nb * nt * slots * n * 2);
+    auto fill = [&](auto* phases, const auto& packed, K kind) {
+        typedef std::remove_const_t<std::remove_pointer_t<decltype(phases)>> T;
+        std::vector<RightItem<T>> v;
+        for (int item = 0; item < nb; ++item)
+            for (int j = 0; j < nt / g; ++j) {
+                const ChainK k = kf(item, j);
+                const double* d0 = ph + (long)item * 2 * nt * n + (long)j * g * n;
+                const T* d = phases + (long)item * 2 * nt * n;
+                v.push_back({packed[item % nspecies]->template as<T>(), k.re, k.re + k.plane, k.ld, k.sign, d0,
+                             d0 + (long)nt * n, d, d + (long)nt * n,
+                             g > 1 ? Suf + ((long)item * nt + j * g + 1) * 2 * nn : nullptr, 2 * nn,
+                             part + ((long)item * nt + j * g) * slots * n * 2, j * g, g});
+            }
+        b.add(kind, v, n, n);
+    };
+    if (ph32)
+        fill(ph32, pk32_, K::RIGHT32);
+    else
+        fill(ph, pk64_, K::RIGHT64);
+    std::vector<DReduceItem> dr;
+    for (int item = 0; item < nb; ++item)
+        for (int tau = 0; tau < nt; ++tau)
+            dr.push_back({part + ((long)item * nt + tau) * slots * n * 2, ((long)item * nt + tau) * n, n, slots});
+    b.add(K::DREDUCE, dr);
+    op.direct = true;
+}
+
 // ---------------------------------------------------------------------------
-void Plan::run(OpCache& op, const double* phi) {
+void Plan::run(OpCache& op, const double* phi, double* out) {
     for (const Step& st : op.steps)
-        if (!launch_step(op, st, phi)) throw std::runtime_error("a step's launch shape does not fit it");
+        if (!launch_step(op, st, phi, out)) throw std::runtime_error("a step's launch shape does not fit it");
 }
 
 void Plan::set_tile(int kind, int tile) {
@@ -397,8 +603,8 @@ void Plan::tune(OpCache& op) {
 
 void Plan::profile(const double* phi, int opk, int nt, int batch, int group, int nspecies, int spin, int reps,
                    double* out, int nkinds) {
-    OpCache& op = opk == 0   ? get_force_plain(nt, batch, nspecies, spin)
-                  : opk == 1 ? get_force_mixed(nt, batch, group, nspecies, spin)
+    OpCache& op = opk == 0   ? get_force(0, nt, batch, group, nspecies, spin)
+                  : opk == 1 ? get_force(1, nt, batch, group, nspecies, spin)
                   : opk == 2 ? get_logdet_plain(nt, batch, nspecies, spin)
                   : opk == 3 ? get_logdet_grouped(nt, batch, group, nspecies, spin)
                   : opk == 4 ? get_force_stable(nt, batch, group, nspecies, spin)
@@ -433,7 +639,7 @@ void Plan::profile(const double* phi, int opk, int nt, int batch, int group, int
     }
 }
 
-bool Plan::launch_step(OpCache& op, const Step& st, const double* phi) {
+bool Plan::launch_step(OpCache& op, const Step& st, const double* phi, double* out) {
     const int n = nx_;
     const long nn = (long)n * n;
     hipStream_t s = stream_;
@@ -557,7 +763,16 @@ bool Plan::launch_step(OpCache& op, const Step& st, const double* phi) {
             break;
         case K::DREDUCE:
             hipLaunchKernelGGL(diag_reduce_kernel, dim3(cdiv(n, 256), st.count), dim3(256), 0, s,
-                               (const DReduceItem*)st.items);
+                               (const DReduceItem*)st.items, out ? out : op.parts);
+            break;
+        case K::SUFFIX64:
+            launch_suffix_chain((const SuffixItem*)st.items, st.count, n, s);
+            break;
+        case K::RIGHT32:
+            launch_right_chain<float>((const RightItem<float>*)st.items, st.count, n, s);
+            break;
+        case K::RIGHT64:
+            launch_right_chain<double>((const RightItem<double>*)st.items, st.count, n, s);
             break;
         case K::RGATHER:
             hipLaunchKernelGGL(row_gather_kernel, dim3(std::min<int>(cdiv(st.aux, 256), 64), st.max_m, st.count), dim3(256),
@@ -720,7 +935,7 @@ OpCache& Plan::get_force_plain(int nt, int batch, int nspecies, int spin) {
 // (g/k + k + 1) instead of g stored suffix matrices.
 OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin) {
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
-    const int ck = (recompute_ > 0 && recompute_ < g && g % recompute_ == 0 && nx_ % 32 == 0) ? recompute_ : 0;
+    const int ck = recomputes(g) ? recompute_ : 0;
     auto key = std::make_tuple(1 + 16 * ck, nt, batch, g, nspecies, spin);
     auto found = cache_.find(key);
     if (found != cache_.end()) return *found->second;
@@ -744,12 +959,7 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
     double* Suf = b.d64((size_t)nb * ng * suf_per_group * 2 * nn);
     // right chains: every product, or the last two per group when the diagonal is fused
     float* Rt = b.d32((size_t)nb * (fuse ? 2 * ng : nt) * 2 * nn);
-    double* GL = b.d64((size_t)nb * ng * 2 * nn);
-    double* RR = b.d64((size_t)nb * ng * 2 * nn);
-    double* KK = b.d64((size_t)nb * ng * 2 * nn);
     float* K32 = b.d32((size_t)nb * ng * 2 * nn);
-    double* LUb = b.d64((size_t)nb * 2 * nn);
-    int* piv = b.di((size_t)nb * n);
     op->parts = b.d64((size_t)nb * nt * n * 2);
     auto D = [&](int item, int t) { return CMat<float>{ph + (long)item * 2 * nt * n + (long)t * n,
                                                        ph + (long)item * 2 * nt * n + (long)nt * n + (long)t * n}; };
@@ -779,7 +989,6 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
     auto mRt = [&](int item, int t) {
         return fuse ? cmat(Rt, ((long)item * ng + t / g) * 2 + (t & 1), nn) : cmat(Rt, (long)item * nt + t, nn);
     };
-    auto m64 = [&](double* base, int item, int j) { return cmat(base, (long)item * ng + j, nn); };
     auto mP = [&](int item, int j) { return mS(item, j * g); };  // group product P_j = Suf_{s_j}
     auto mK32 = [&](int item, int j) { return cmat(K32, (long)item * ng + j, nn); };
     auto spec = [&](int item) { return item % nspecies; };
@@ -815,97 +1024,7 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
         b.add(K::GEMM64_RC_ROW, gi, n, n);
     }
     // ---- top level (FP64)
-    if (ng == 1) {
-        std::vector<CopyItem<double, double>> cp;
-        for (int item = 0; item < nb; ++item) cp.push_back({mP(item, 0).re, LUb + (long)item * 2 * nn, 2 * nn});
-        b.add(K::COPY64, cp, (int)(2 * nn));
-    } else {
-        std::vector<CopyItem<double, double>> cp;
-        for (int item = 0; item < nb; ++item) cp.push_back({mP(item, ng - 1).re, m64(GL, item, ng - 2).re, 2 * nn});
-        b.add(K::COPY64, cp, (int)(2 * nn));
-        for (int j = ng - 3; j >= 0; --j) {
-            std::vector<GemmItem<double>> gi;
-            for (int item = 0; item < nb; ++item) {
-                const CMat<double> a = mP(item, j + 1), bb = m64(GL, item, j + 1);
-                gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(GL, item, j), nullptr, nullptr, nullptr,
-                                           nullptr, n));
-            }
-            b.add(K::GEMM64_CC, gi, n, n);
-        }
-        std::vector<GemmItem<double>> gi;
-        for (int item = 0; item < nb; ++item) {
-            const CMat<double> a = mP(item, 0), bb = m64(GL, item, 0);
-            gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, cmat(LUb, item, nn), nullptr, nullptr, nullptr,
-                                       nullptr, n));
-        }
-        b.add(K::GEMM64_CC, gi, n, n);
-    }
-    {
-        std::vector<LuItem> lu;
-        double* luw = b.d64(nb * lu_work_doubles(n));
-        for (int item = 0; item < nb; ++item)
-            lu.push_back({LUb + (long)item * 2 * nn, LUb + (long)item * 2 * nn + nn, piv + (long)item * n, nullptr,
-                          luw + item * lu_work_doubles(n), n, n});
-        b.add(K::LU, lu, n, 0, 1);
-        if (n % LU_NB == 0) {
-            // Mid = (1 + P_0 GL_0)^{-1} = U^{-1} L^{-1} P: the row-permuted identity, then two
-            // blocked triangular solves on GEMMs
-            int* sig = b.di((size_t)nb * n);
-            double* S1 = b.d64((size_t)nb * 2 * nn);
-            double* S2 = b.d64((size_t)nb * 2 * nn);
-            std::vector<SigmaItem> sv;
-            std::vector<GatherItem> ga;
-            std::vector<TrsmMat> tl, tu;
-            for (int item = 0; item < nb; ++item) {
-                const CMat<double> s1 = cmat(S1, item, nn), s2 = cmat(S2, item, nn), rr = m64(RR, item, 0);
-                const double* fre = LUb + (long)item * 2 * nn;
-                sv.push_back({piv + (long)item * n, sig + (long)item * n, n, n});
-                ga.push_back({sig + (long)item * n, nullptr, nullptr, s1.re, s1.im, nullptr, nullptr, n, n, n, n, 0});
-                tl.push_back({fre, fre + nn, n, luw + item * lu_work_doubles(n), s1.re, s1.im, n, s2.re, s2.im, n});
-                tu.push_back({fre, fre + nn, n, luw + item * lu_work_doubles(n), s2.re, s2.im, n, rr.re, rr.im, n});
-            }
-            b.add(K::SIGMA, sv);
-            b.add(K::GATHER, ga, n, 0, 0, n);
-            add_trsm(b, 0, n, n, tl);
-            add_trsm(b, 1, n, n, tu);
-        } else {
-            std::vector<SolveItem> sv;
-            for (int item = 0; item < nb; ++item) {
-                SolveItem si{};
-                si.lu_re = LUb + (long)item * 2 * nn;
-                si.lu_im = si.lu_re + nn;
-                si.piv = piv + (long)item * n;
-                si.dinv = luw + item * lu_work_doubles(n);
-                si.x_re = m64(RR, item, 0).re;
-                si.x_im = m64(RR, item, 0).im;
-                si.xsr = n;
-                si.xsc = 1;
-                si.n = n;
-                si.ld = n;
-                si.nrhs = n;
-                sv.push_back(si);
-            }
-            b.add(K::SOLVE, sv, n, n);
-        }
-    }
-    for (int j = 1; j < ng; ++j) {
-        std::vector<GemmItem<double>> gi;
-        for (int item = 0; item < nb; ++item) {
-            const CMat<double> a = m64(RR, item, j - 1), bb = mP(item, j - 1);
-            gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(RR, item, j), nullptr, nullptr, nullptr, nullptr, n));
-        }
-        b.add(K::GEMM64_CC, gi, n, n);
-    }
-    if (ng > 1) {
-        std::vector<GemmItem<double>> gi;
-        for (int item = 0; item < nb; ++item)
-            for (int j = 0; j < ng - 1; ++j) {
-                const CMat<double> a = m64(GL, item, j), bb = m64(RR, item, j);
-                gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(KK, item, j), nullptr, nullptr, nullptr,
-                                           nullptr, n));
-            }
-        b.add(K::GEMM64_CC, gi, n, n);
-    }
+    const TopLevel tl = add_top_level(b, n, ng, nb, mP, n % LU_NB == 0);
     // ---- local right chains (FP32), transposed.  With n % 32 == 0 the chain products also
     //      produce the force diagonal f[tau] = rowdot(Suf_{tau+1}, Rt_tau) (diag Rt at a group's
     //      last slice) as partial row sums per 16 columns, summed by one reduction at the end,
@@ -922,7 +1041,7 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
         std::vector<ColScaleItem> cv;
         for (int item = 0; item < nb; ++item)
             for (int j = 0; j < ng; ++j) {
-                const double* src = (j < ng - 1) ? m64(KK, item, j).re : m64(RR, item, ng - 1).re;
+                const double* src = tl.k(item, j);
                 cv.push_back({src, src + nn, n, 1.0, mK32(item, j).re, D64(item, j * g).re, D64(item, j * g).im, n});
             }
         b.add(K::COLSCALE64TO32, cv);
@@ -930,7 +1049,7 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
         std::vector<TCopyItem<double, float>> cv;
         for (int item = 0; item < nb; ++item)
             for (int j = 0; j < ng; ++j) {
-                const double* src = (j < ng - 1) ? m64(KK, item, j).re : m64(RR, item, ng - 1).re;
+                const double* src = tl.k(item, j);
                 cv.push_back({src, mK32(item, j).re, n});
             }
         b.add(K::TCVT64TO32, cv);
@@ -991,9 +1110,9 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
         std::vector<DReduceItem> dr;
         for (int item = 0; item < nb; ++item)
             for (int tau = 0; tau < nt; ++tau)
-                dr.push_back({part + ((long)item * nt + tau) * slots * n * 2, op->parts + ((long)item * nt + tau) * 2 * n,
-                              n, slots});
+                dr.push_back({part + ((long)item * nt + tau) * slots * n * 2, ((long)item * nt + tau) * n, n, slots});
         b.add(K::DREDUCE, dr);
+        op->direct = true;
     } else {
         std::vector<DiagItem<double, float>> dg;
         for (int item = 0; item < nb; ++item)
@@ -1012,6 +1131,46 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
     return ref;
 }
 
+// The grouped force on the strip kernels (chain.hpp): every group's suffix chain in one launch,
+// the top level, every group's right chain with the diagonal fused in one launch.  right32: the
+// mixed form (FP32 right chains); else FP64 throughout.
+OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin, bool right32) {
+    if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
+    auto key = std::make_tuple(right32 ? 1 : 0, nt, batch, g, nspecies, spin);
+    auto found = cache_.find(key);
+    if (found != cache_.end()) return *found->second;
+    auto op = std::make_unique<OpCache>();
+    op->nt = nt;
+    op->batch = batch;
+    op->nspecies = nspecies;
+    op->phi_stride = 2L * nx_ * nt;
+    Builder b(*op);
+    const int n = nx_, nb = batch * nspecies, ng = nt / g;
+    const long nn = (long)n * n;
+    double* ph = b.d64((size_t)nb * 2 * nt * n);
+    float* ph32 = right32 ? b.d32((size_t)nb * 2 * nt * n) : nullptr;
+    double* Suf = b.d64((size_t)nb * nt * 2 * nn + 32 * (size_t)n);
+    op->parts = b.d64((size_t)nb * nt * n * 2);
+    auto mS = [&](int item, int t) { return cmat(Suf, (long)item * nt + t, nn); };
+    std::vector<PhaseItem> phs;
+    for (int item = 0; item < nb; ++item) {
+        double* d = ph + (long)item * 2 * nt * n;
+        float* d32 = right32 ? ph32 + (long)item * 2 * nt * n : nullptr;
+        phs.push_back({item / nspecies, spin, sigma_of(item % nspecies), d, d + (long)nt * n, d32,
+                       right32 ? d32 + (long)nt * n : nullptr, n, nt});
+    }
+    b.add(K::PHASE, phs);
+    add_suffix(b, nt, g, nb, nspecies, ph, [&](int item, int j) { return mS(item, j * g + g - 1).re; }, -2 * nn, 1);
+    const TopLevel tl = add_top_level(b, n, ng, nb, [&](int item, int j) { return mS(item, j * g); },
+                                      n % LU_NB == 0 && nb > 4);
+    add_right(b, *op, nt, g, nb, nspecies, ph, ph32, Suf, [&](int item, int j) { return ChainK{tl.k(item, j), nn, n, 1.0}; });
+    b.finish();
+    tune(*op);
+    auto& ref = *op;
+    cache_[key] = std::move(op);
+    return ref;
+}
+
 // ---------------------------------------------------------------------------
 // Plain FP64 logdetM, the reference's chains (hubbardFermiMatrixExp.cpp:574-612,
 // hubbardFermiMatrixDia.cpp:571-597):
@@ -1020,6 +1179,8 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
 //                   auxT <- A_s (D_t auxT), auxT_0 = A_s D_0;  det(1 + aux) = det(1 + auxT)
 //   then LU of (1 + .) with its log-determinant.
 OpCache& Plan::get_logdet_plain(int nt, int batch, int nspecies, int spin) {
+    if (chain_fits(nx_))
+        return get_logdet_chains(nt, batch, nt, nspecies, spin, true);
     auto key = std::make_tuple(2, nt, batch, 0, nspecies, spin);
     auto found = cache_.find(key);
     if (found != cache_.end()) return *found->second;
@@ -1087,6 +1248,7 @@ OpCache& Plan::get_logdet_plain(int nt, int batch, int nspecies, int spin) {
 // for all groups in parallel, then A^{-1} = P_0 ... P_{ng-1}, then LU of 1 + A^{-1}.
 OpCache& Plan::get_logdet_grouped(int nt, int batch, int g, int nspecies, int spin) {
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
+    if (chain_fits(nx_)) return get_logdet_chains(nt, batch, g, nspecies, spin, false);
     auto key = std::make_tuple(3, nt, batch, g, nspecies, spin);
     auto found = cache_.find(key);
     if (found != cache_.end()) return *found->second;
@@ -1156,6 +1318,73 @@ OpCache& Plan::get_logdet_grouped(int nt, int batch, int g, int nspecies, int sp
             const CMat<double> last = mT(item, (ng - 2) & 1);
             lu.push_back({last.re, last.im, piv + (long)item * n, op->logdet + 2 * item, work(item), n, n});
         }
+    }
+    b.add(K::LU, lu, n, 0, 1);
+    b.finish();
+    tune(*op);
+    auto& ref = *op;
+    cache_[key] = std::move(op);
+    return ref;
+}
+
+// log det M on the strip kernels: the products of groups of g slices in one launch, multiplied
+// together pairwise (all pairs of a level in one launch), then the LU of 1 + (.).  reference: the
+// chains of the reference's algorithm in its order (see get_logdet_plain); else the inverse form
+// X_0 ... X_{nt-1} for both species.
+OpCache& Plan::get_logdet_chains(int nt, int batch, int g, int nspecies, int spin, bool reference) {
+    if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
+    auto key = std::make_tuple(reference ? 2 : 3, nt, batch, g, nspecies, spin);
+    auto found = cache_.find(key);
+    if (found != cache_.end()) return *found->second;
+    auto op = std::make_unique<OpCache>();
+    op->nt = nt;
+    op->batch = batch;
+    op->nspecies = nspecies;
+    op->phi_stride = 2L * nx_ * nt;
+    Builder b(*op);
+    const int n = nx_, nb = batch * nspecies, ng = nt / g;
+    const long nn = (long)n * n;
+    double* ph = b.d64((size_t)nb * 2 * nt * n);
+    double* W[2] = {b.d64((size_t)nb * ng * 2 * nn), ng > 1 ? b.d64((size_t)nb * ((ng + 1) / 2) * 2 * nn) : nullptr};
+    int* piv = b.di((size_t)nb * n);
+    op->logdet = b.d64((size_t)nb * 2);
+    auto bchain = [&](int item) { return reference && hop_ == EXP && item % nspecies == PARTICLE; };
+    std::vector<PhaseItem> phs;
+    std::vector<SuffixItem> sv;
+    for (int item = 0; item < nb; ++item) {
+        double* d = ph + (long)item * 2 * nt * n;
+        const int s = item % nspecies;
+        const bool fw = bchain(item);
+        phs.push_back({item / nspecies, spin, fw ? 1.0 : sigma_of(s), d, d + (long)nt * n, nullptr, nullptr, n, nt});
+        for (int j = 0; j < ng; ++j)
+            sv.push_back({(fw ? pke64_ : pk64_[s])->as<double>(), (fw ? e64_[s] : a64_[s])->as<double>(), d,
+                          d + (long)nt * n, cmat(W[0], (long)item * ng + j, nn).re, 0,
+                          reference ? j * g : j * g + g - 1, reference ? 1 : -1, g, 0, reference});
+    }
+    b.add(K::PHASE, phs);
+    b.add(K::SUFFIX64, sv, n, n);
+    int k = ng, at = 0;  // k products per item, in W[at]
+    for (; k > 1; k = (k + 1) / 2, at ^= 1) {
+        std::vector<GemmItem<double>> gi;
+        std::vector<CopyItem<double, double>> cp;
+        const int h = (k + 1) / 2;
+        for (int item = 0; item < nb; ++item) {
+            auto src = [&](int j) { return cmat(W[at], (long)item * k + j, nn); };
+            for (int j = 0; j + 1 < k; j += 2) {
+                const CMat<double> l = src(reference ? j + 1 : j), r = src(reference ? j : j + 1);
+                gi.push_back(gitem<double>(l.re, l.im, r.re, r.im, cmat(W[at ^ 1], (long)item * h + j / 2, nn), nullptr,
+                                           nullptr, nullptr, nullptr, n));
+            }
+            if (k % 2) cp.push_back({src(k - 1).re, cmat(W[at ^ 1], (long)item * h + h - 1, nn).re, 2 * nn});
+        }
+        b.add(K::GEMM64_CC, gi, n, n);
+        b.add(K::COPY64, cp, (int)(2 * nn));
+    }
+    std::vector<LuItem> lu;
+    double* luw = b.d64(nb * lu_work_doubles(n));
+    for (int item = 0; item < nb; ++item) {
+        const CMat<double> m = cmat(W[at], item, nn);
+        lu.push_back({m.re, m.im, piv + (long)item * n, op->logdet + 2 * item, luw + item * lu_work_doubles(n), n, n});
     }
     b.add(K::LU, lu, n, 0, 1);
     b.finish();
@@ -1314,7 +1543,8 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
     const long nn = (long)n * n;
     const int nb = batch * nspecies;
     double* ph = b.d64((size_t)nb * 2 * nt * n);
-    double* Wg = b.d64((size_t)nb * ng * 2 * 2 * nn);
+    const bool chains = chain_fits(n);
+    double* Wg = b.d64((size_t)nb * ng * (chains ? 1 : 2) * 2 * nn);  // P_j, or two products in turn
     op->logdet = b.d64((size_t)nb * (ng - 1) * 2);
     auto D = [&](int item, int t) { return CMat<double>{ph + (long)item * 2 * nt * n + (long)t * n,
                                                         ph + (long)item * 2 * nt * n + (long)nt * n + (long)t * n}; };
@@ -1324,15 +1554,19 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
     for (int item = 0; item < nb; ++item)
         phs.push_back({item / nspecies, spin, sigma_of(spec(item)), D(item, 0).re, D(item, 0).im, nullptr, nullptr, n, nt});
     b.add(K::PHASE, phs);
+    auto P = [&](int item, int j) {
+        return chains ? cmat(Wg, (long)item * ng + j, nn) : mW(item, j, (g - 1) & 1);
+    };
+    if (chains) add_suffix(b, nt, g, nb, nspecies, ph, [&](int item, int j) { return P(item, j).re; }, 0, 0);
     std::vector<ScaleItem<double>> sc;
-    for (int item = 0; item < nb; ++item)
+    for (int item = 0; item < nb && !chains; ++item)
         for (int j = 0; j < ng; ++j) {
             const int e = j * g + g - 1;
             sc.push_back({a64_[spec(item)]->as<double>(), D(item, e).re, D(item, e).im, mW(item, j, 0).re,
                           mW(item, j, 0).im, n, SCALE_ROW});
         }
     b.add(K::SCALE64, sc);
-    for (int q = 1; q < g; ++q) {
+    for (int q = 1; q < g && !chains; ++q) {
         std::vector<GemmItem<double>> gi;
         for (int item = 0; item < nb; ++item)
             for (int j = 0; j < ng; ++j) {
@@ -1343,7 +1577,7 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
             }
         b.add(K::GEMM64_RC_ROW, gi, n, n);
     }
-    add_cyclic_factor(b, n, ng, nb, [&](int item, int j) { return mW(item, j, (g - 1) & 1); }, op->logdet);
+    add_cyclic_factor(b, n, ng, nb, P, op->logdet);
     b.finish();
     tune(*op);
     auto& ref = *op;
@@ -1377,11 +1611,12 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
     const long wd = (long)ng * n;  // columns of the block solves
     double* ph = b.d64((size_t)nb * 2 * nt * n);
     float* ph32 = right32 ? b.d32((size_t)nb * 2 * nt * n) : nullptr;
-    double* Suf = b.d64((size_t)nb * nt * 2 * nn);
-    double* Rt = right32 ? nullptr : b.d64((size_t)nb * nt * 2 * nn);
-    float* Rt32 = right32 ? b.d32((size_t)nb * ng * 2 * 2 * nn) : nullptr;  // last two products per group
-    double* Kt = right32 ? nullptr : b.d64((size_t)nb * ng * 2 * nn);
-    float* K32 = right32 ? b.d32((size_t)nb * ng * 2 * nn) : nullptr;
+    double* Suf = b.d64((size_t)nb * nt * 2 * nn + 32 * (size_t)n);
+    const bool chains = chain_fits(n);
+    double* Rt = right32 || chains ? nullptr : b.d64((size_t)nb * nt * 2 * nn);
+    float* Rt32 = right32 && !chains ? b.d32((size_t)nb * ng * 2 * 2 * nn) : nullptr;  // last two products per group
+    double* Kt = right32 || (chains && ng > 1) ? nullptr : b.d64((size_t)nb * ng * 2 * nn);
+    float* K32 = right32 && !chains ? b.d32((size_t)nb * ng * 2 * nn) : nullptr;
     double* Tb = b.d64((size_t)nb * ng * 2 * n * wd);
     op->parts = b.d64((size_t)nb * nt * n * 2);
     auto D = [&](int item, int t) {
@@ -1404,7 +1639,9 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
         phs.push_back({item / nspecies, spin, sigma_of(spec(item)), D(item, 0).re, D(item, 0).im,
                        right32 ? D32(item, 0).re : nullptr, right32 ? D32(item, 0).im : nullptr, n, nt});
     b.add(K::PHASE, phs);
-    {
+    if (chains)
+        add_suffix(b, nt, g, nb, nspecies, ph, [&](int item, int j) { return mS(item, j * g + g - 1).re; }, -2 * nn, 1);
+    if (!chains) {
         std::vector<ScaleItem<double>> sc;
         for (int item = 0; item < nb; ++item)
             for (int j = 0; j < ng; ++j) {
@@ -1414,7 +1651,7 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
             }
         b.add(K::SCALE64, sc);
     }
-    for (int q = 1; q < g; ++q) {
+    for (int q = 1; q < g && !chains; ++q) {
         std::vector<GemmItem<double>> gi;
         for (int item = 0; item < nb; ++item)
             for (int j = 0; j < ng; ++j) {
@@ -1462,8 +1699,8 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
             si.dinv = luw + item * lu_work_doubles(n);
             si.x_re = mK(item, 0).re;
             si.x_im = mK(item, 0).im;
-            si.xsr = 1;  // written transposed: K^T
-            si.xsc = n;
+            si.xsr = chains ? n : 1;  // K, or K^T for the chain products
+            si.xsc = chains ? 1 : n;
             si.n = n;
             si.ld = n;
             si.nrhs = n;
@@ -1549,7 +1786,9 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
             b.add(K::BLOCK, cp, 0, 0, 0, n * w);
             add_trsm(b, 1, n, w, tu);
         }
-        if (right32) {
+        if (chains) {
+            // the right chains read K_j = -X[j+1][j] (X[0][ng-1] for the last group) in place
+        } else if (right32) {
             // K_j = sign X (untransposed) to FP32 with the group's first phase: K_j D_{s_j}
             std::vector<ColScaleItem> cv;
             for (int item = 0; item < nb; ++item)
@@ -1571,6 +1810,18 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
                 }
             b.add(K::TBLOCK, tb);
         }
+    }
+    if (chains) {
+        add_right(b, *op, nt, g, nb, nspecies, ph, ph32, Suf, [&](int item, int j) {
+            if (ng == 1) return ChainK{mK(item, 0).re, nn, n, 1.0};
+            const CMat<double> x = j < ng - 1 ? mT(item, j + 1) : mT(item, 0);
+            return ChainK{x.re + (j < ng - 1 ? (long)(j + 1) * n : 0), (long)n * wd, wd, j < ng - 1 ? -1.0 : 1.0};
+        });
+        b.finish();
+        tune(*op);
+        auto& ref = *op;
+        cache_[key] = std::move(op);
+        return ref;
     }
     if (right32) {
         // ---- local right chains in FP32 on MFMA with the force diagonal fused (as in the
@@ -1602,9 +1853,9 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
         std::vector<DReduceItem> dr;
         for (int item = 0; item < nb; ++item)
             for (int tau = 0; tau < nt; ++tau)
-                dr.push_back({part + ((long)item * nt + tau) * slots * n * 2, op->parts + ((long)item * nt + tau) * 2 * n,
-                              n, slots});
+                dr.push_back({part + ((long)item * nt + tau) * slots * n * 2, ((long)item * nt + tau) * n, n, slots});
         b.add(K::DREDUCE, dr);
+        op->direct = true;
         b.finish();
         tune(*op);
         auto& ref = *op;
@@ -1683,8 +1934,38 @@ void Plan::logdetM(const double* phi, int nt, int batch, int mode, int group, in
     }
 }
 
+// Slices per group of the plain FP64 force for nb (field, species) items: one chain over all
+// slices (the reference's own order of products), or, for lattices beyond the register-resident
+// strip kernels (n > CHAIN_MAX_RES), the grouping with the shortest time where few items leave the
+// GPU idle.  Times in MFMA cycles of a SIMD: a slice takes its tiles' products (32 n each) and
+// about 900 cycles of latency, a top-level product (2 ng - 1 of them in sequence) about 7000 cycles
+// and its share of n^3.  One field at n = 288, Nt = 96: 6.4 ms with one group, 2.06 ms with six.
+int Plan::plain_group(int nt, int nb) const {
+    const int n = nx_, tiles = chain_tiles(n);
+    if (n <= CHAIN_MAX_RES) return nt;
+    int best = nt;
+    double cost = 0;
+    for (int ng = 1; ng <= std::max(1, nt / 4); ++ng) {
+        if (nt % ng != 0) continue;
+        const long t1 =
+            chain_cost(CHAIN_SHAPES[chain_shape<double>(n, nb * ng, CHAIN_CUS)], tiles, nb * ng, CHAIN_CUS);
+        const double slice = t1 * 32.0 * n * 1.15 + 900.0;
+        const double product = 7000.0 + 0.0016 * n * (double)n * n * std::max(1.0, nb / 8.0);
+        const double c = 2.0 * (nt / ng) * slice + (ng > 1 ? (2 * ng - 1) * product : 0.0);
+        if (ng == 1 || c < 0.95 * cost) {
+            cost = c;
+            best = nt / ng;
+        }
+    }
+    return best;
+}
+
 OpCache& Plan::get_force(int mode, int nt, int batch, int group, int nspecies, int spin) {
     if (nt < 2) throw std::invalid_argument("nt < 2 in HubbardFermiAction algorithm DIRECT_SINGLE not supported");
+    if (chain_fits(nx_)) {
+        if (mode == 0) return get_force_chains(nt, batch, plain_group(nt, batch * nspecies), nspecies, spin, false);
+        if (mode == 1 && !recomputes(group)) return get_force_chains(nt, batch, group, nspecies, spin, true);
+    }
     return mode == 0   ? get_force_plain(nt, batch, nspecies, spin)
            : mode == 1 ? get_force_mixed(nt, batch, group, nspecies, spin)
                        : get_force_stable(nt, batch, group, nspecies, spin, mode == 3);
@@ -1693,7 +1974,8 @@ OpCache& Plan::get_force(int mode, int nt, int batch, int group, int nspecies, i
 void Plan::force_parts(const double* phi, int nt, int batch, int mode, int group, int nspecies, int spin,
                        double* out_dev) {
     OpCache& op = get_force(mode, nt, batch, group, nspecies, spin);
-    run(op, phi);
+    run(op, phi, op.direct ? out_dev : nullptr);
+    if (op.direct) return;
     const size_t bytes = (size_t)batch * nspecies * nt * nx_ * 2 * 8;
     ISLE_HIP(hipMemcpyAsync(out_dev, op.parts, bytes, hipMemcpyDeviceToDevice, stream_));
 }
@@ -1702,7 +1984,7 @@ void Plan::force_parts(const double* phi, int nt, int batch, int mode, int group
 // steps; operations share nothing but read-only slice matrices, so any interleaving that
 // keeps every operation's own order is correct.  Two steps can share a launch when they have
 // the same kind, descriptor size and launch parameters (GEMM kinds: any m, n, the launch
-// covers the largest) and neither binds the caller's fields (PHASE).  The sequences are
+// covers the largest) and neither binds the caller's arrays (PHASE, DREDUCE).  The sequences are
 // merged one after another into a shortest common supersequence under that relation (dynamic
 // programming over the two sequences), so the merged operation has as few launches as that
 // greedy order allows; each merged step's descriptors are the concatenation of its members'.
@@ -1715,7 +1997,7 @@ std::unique_ptr<Plan::MultiOp> Plan::merge_ops(const std::vector<OpCache*>& ops)
     };
     auto step_of = [&](const Member& mb) -> const Step& { return ops[mb.op]->steps[mb.step]; };
     auto joinable = [&](const Step& a, const Step& b) {
-        if (a.kind != b.kind || a.kind == K::PHASE || a.ibytes != b.ibytes || a.flag != b.flag || a.aux != b.aux)
+        if (a.kind != b.kind || a.kind == K::PHASE || a.kind == K::DREDUCE || a.ibytes != b.ibytes || a.flag != b.flag || a.aux != b.aux)
             return false;
         return is_gemm(a.kind) || (a.max_m == b.max_m && a.max_n == b.max_n);
     };
@@ -1781,7 +2063,7 @@ std::unique_ptr<Plan::MultiOp> Plan::merge_ops(const std::vector<OpCache*>& ops)
         const Slot& sl = seq[q];
         Step st = step_of(sl.members[0]);
         if (sl.members.size() == 1) {  // the member's own descriptors and launch
-            mo->owner.push_back(st.kind == K::PHASE ? sl.members[0].op : -1);
+            mo->owner.push_back(st.kind == K::PHASE || st.kind == K::DREDUCE ? sl.members[0].op : -1);
             mo->merged.steps.push_back(st);
             continue;
         }
@@ -1833,10 +2115,11 @@ void Plan::force_parts_multi(int nops, const double* const* phis, const int* nts
     for (size_t q = 0; q < mo->merged.steps.size(); ++q) {
         const int o = mo->owner[q];
         const Step& st = mo->merged.steps[q];
-        const bool ok = o >= 0 ? launch_step(*mo->ops[o], st, phis[o]) : launch_step(mo->merged, st, nullptr);
+        const bool ok = o >= 0 ? launch_step(*mo->ops[o], st, phis[o], outs[o]) : launch_step(mo->merged, st, nullptr);
         if (!ok) throw std::runtime_error("a step's launch shape does not fit it");
     }
     for (int i = 0; i < nops; ++i) {
+        if (mo->ops[i]->direct) continue;
         const size_t bytes = (size_t)batches[i] * nspecies * nts[i] * nx_ * 2 * 8;
         ISLE_HIP(hipMemcpyAsync(outs[i], mo->ops[i]->parts, bytes, hipMemcpyDeviceToDevice, stream_));
     }

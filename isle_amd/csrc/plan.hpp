@@ -10,6 +10,7 @@
 #include <tuple>
 #include <vector>
 
+#include "chain.hpp"
 #include "common.hpp"
 #include "cyclic.hpp"
 #include "elementwise.hpp"
@@ -73,6 +74,8 @@ enum class K : int {
     LU_SHAPE_DEFER,     // LU_SHAPE whose columns beyond kf take the row interchanges only
     GEMM64_CC4,         // complex x complex with four real products       (f64)
     GEMM64_CC4_SUB,     // C -= A B, the same                              (f64)
+    SUFFIX64,           // whole suffix chains on column strips (chain.hpp) (f64)
+    RIGHT32, RIGHT64,   // whole right chains with the force diagonal fused (f32, f64)
     KIND_END
 };
 
@@ -98,10 +101,13 @@ struct OpCache {
     long phi_stride = 0;       // doubles between consecutive fields of the batch
     double* logdet = nullptr;  // device [batch][nspecies][2]
     double* parts = nullptr;   // device [batch][nspecies][nx*nt] interleaved
+    bool direct = false;       // the last step (DREDUCE) writes the parts to the caller's array
     int nspecies = 0;
     int batch = 0;
     int nt = 0;
 };
+
+struct Builder;
 
 class Plan {
 public:
@@ -179,6 +185,8 @@ private:
     std::map<int, int> forced_;  // kind -> pinned tile
     // inverse-form slice matrices A_s (EXP: exp(-k+mu), exp(-s k-mu); DIA: K_p, K_h)
     std::unique_ptr<DevBuf> a64_[2], a32_[2];
+    // the same in the operand order of the strip kernels (chain.hpp), where they take this order
+    std::unique_ptr<DevBuf> pk64_[2], pk32_[2], pke64_;  // pke64_: exp(k-mu) of the particles
     // EXP non-inverse matrices exp(k-mu), exp(s k+mu)
     std::unique_ptr<DevBuf> e64_[2];
     double logdet_a_[2] = {0, 0};
@@ -205,14 +213,25 @@ private:
     void build_exp(const std::vector<double>& x, DevBuf& out);
     OpCache& get_force_plain(int nt, int batch, int nspecies, int spin);
     OpCache& get_force_mixed(int nt, int batch, int group, int nspecies, int spin);
+    bool recomputes(int g) const {
+        return recompute_ > 0 && recompute_ < g && g % recompute_ == 0 && nx_ % 32 == 0;
+    }
+    int plain_group(int nt, int nb) const;
+    template <typename OF>
+    void add_suffix(Builder& b, int nt, int g, int nb, int nspecies, const double* ph, OF out, long step, int all);
+    template <typename KF>
+    void add_right(Builder& b, OpCache& op, int nt, int g, int nb, int nspecies, const double* ph, const float* ph32,
+                   const double* Suf, KF kf);
+    OpCache& get_force_chains(int nt, int batch, int group, int nspecies, int spin, bool right32);
     OpCache& get_logdet_plain(int nt, int batch, int nspecies, int spin);
+    OpCache& get_logdet_chains(int nt, int batch, int g, int nspecies, int spin, bool reference);
     OpCache& get_logdet_grouped(int nt, int batch, int group, int nspecies, int spin);
     OpCache& get_force_stable(int nt, int batch, int group, int nspecies, int spin, bool right32 = false);
     OpCache& get_logdet_stable(int nt, int batch, int group, int nspecies, int spin);
     OpCache& get_qlu(int nt);
     OpCache& get_solveq(int nt, int nrhs);
-    void run(OpCache& op, const double* phi);
-    bool launch_step(OpCache& op, const Step& st, const double* phi);
+    void run(OpCache& op, const double* phi, double* out = nullptr);
+    bool launch_step(OpCache& op, const Step& st, const double* phi, double* out = nullptr);
     // Autotuner: time every tile shape of each GEMM step once per (kind, m, n, items) and
     // keep the fastest for that step.
     void tune(OpCache& op);
