@@ -134,6 +134,44 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long k)
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// a_j += m b_j for complex a_j, b_j, j = 0 .. 3, with b_j taken from lane J + j of the 16 lanes that share
+// lane / 16 (a DPP operand: no instruction and no LDS read for the broadcast): a_r += -m_r b_r, then
+// + m_i b_i; nmr = -m_r, nmi = -m_i, mi = m_i.  Every lane of the wave must be active.  The s_nop
+// covers the two wait states between a VALU write of b (a copy the compiler may place) and its DPP read.
+template <int J>
+__device__ __forceinline__ void bcast_fma4(double* ar, double* ai, double br, double bi, double nmr, double mi,
+                                           double nmi) {
+#define ISLE_BCAST(RE, IM, LANE)                                                            \
+    "v_fmac_f64_dpp " RE ", %8, %10 row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t"   \
+    "v_fmac_f64_dpp " RE ", %9, %11 row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t"   \
+    "v_fmac_f64_dpp " IM ", %9, %10 row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t"   \
+    "v_fmac_f64_dpp " IM ", %8, %12 row_newbcast:" LANE " row_mask:0xf bank_mask:0xf\n\t"
+    asm volatile("s_nop 4\n\t" ISLE_BCAST("%0", "%4", "%13") ISLE_BCAST("%1", "%5", "%14")
+                     ISLE_BCAST("%2", "%6", "%15") ISLE_BCAST("%3", "%7", "%16")
+                 : "+v"(ar[0]), "+v"(ar[1]), "+v"(ar[2]), "+v"(ar[3]), "+v"(ai[0]), "+v"(ai[1]), "+v"(ai[2]),
+                   "+v"(ai[3])
+                 : "v"(br), "v"(bi), "v"(nmr), "v"(mi), "v"(nmi), "n"(J), "n"(J + 1), "n"(J + 2), "n"(J + 3));
+#undef ISLE_BCAST
+}
+template <int J0>
+__device__ __forceinline__ void bcast_fma8(double* ar, double* ai, double br, double bi, double nmr, double mi,
+                                           double nmi) {
+    bcast_fma4<J0>(ar, ai, br, bi, nmr, mi, nmi);
+    bcast_fma4<J0 + 4>(ar + 4, ai + 4, br, bi, nmr, mi, nmi);
+}
+
+// 16-byte global accesses, and a wave's own LDS traffic in order (one wave writes and reads: no barrier)
+__device__ __forceinline__ double2 ld_global2(const double* p) {
+    typedef double dbl2 __attribute__((ext_vector_type(2)));
+    const dbl2 v = *(__attribute__((address_space(1))) const dbl2*)p;
+    return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ void st_global2(double* p, double2 v) {
+    typedef double dbl2 __attribute__((ext_vector_type(2)));
+    *(__attribute__((address_space(1))) dbl2*)p = dbl2{v.x, v.y};
+}
+__device__ __forceinline__ void lu_wave_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // L11^{-1} and U11^{-1} of a factorised panel by recursive doubling (lt: L11 unit lower,
 // ut: U11 with its diagonal already inverted, both [NB][NB + 1] in LDS, tl / tu temporaries),
 // then written to the panel's slots of the work buffer.  Ends with a barrier-free copy; the
@@ -235,25 +273,35 @@ __device__ inline void lu_panel_logdet(const LuItem& it, int k0, int nb, int kf,
     }
 }
 
+// Rows of a wave between row-per-lane registers and coalesced memory accesses: a wave's 64 rows of
+// LU_TC columns of one plane in LDS, padded to 16 bytes off a power of two.
+constexpr int LU_TC = 16, LU_TROW = LU_TC + 2;
+
 template <int NB>
 __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __restrict__ items, int k0,
                                                             int add_identity) {
+    constexpr int CG = 8, MAXW = LU_MAX_N / 64;  // columns per group, waves
+    static_assert(NB % LU_TC == 0 && NB % CG == 0, "columns go in groups");
+    constexpr int TRI = NB * (NB + 1);           // one NB x (NB + 1) plane
+    // one after the other: the waves' transposes of the loads, of the stores; then L11 / U11 and the
+    // temporaries of their inversion
+    constexpr int TRANS = MAXW * 64 * LU_TROW;
+    __shared__ __align__(16) double big[TRANS > 8 * TRI ? TRANS : 8 * TRI];
+    __shared__ int pvt[NB];                      // pivot position of each column
     __shared__ unsigned long long pkey[NB];
-    __shared__ int pvt[NB];  // pivot position of each column
-    // the pivot row (re, im pairs); a column's writes and reads are separated by that
-    // column's barriers
-    __shared__ __align__(16) double xrow[2 * NB];
-    __shared__ double lt_re[NB][NB + 1], lt_im[NB][NB + 1];  // L11, inverted in place
-    __shared__ double ut_re[NB][NB + 1], ut_im[NB][NB + 1];  // U11, inverted in place
-    __shared__ double tl_re[NB][NB + 1], tl_im[NB][NB + 1];  // doubling temporaries
-    __shared__ double tu_re[NB][NB + 1], tu_im[NB][NB + 1];
+    __shared__ __align__(16) double2 grow[CG][CG];         // the group's part of its pivot rows
+    __shared__ __align__(16) double2 gu12[CG][NB - CG];    // their rows right of the group
     __shared__ int slot_cnt, slot_dst[2 * NB], slot_src[2 * NB];
-    __shared__ double rsum[LU_MAX_N / 64];
+    __shared__ double rsum[MAXW];
+    // after the column loop: matrix row of each thread's row (80 KB in all: two workgroups on a CU)
+    int* drow = reinterpret_cast<int*>(&gu12[0][0]);
+    static_assert(sizeof(gu12) >= LU_MAX_N * sizeof(int), "row numbers in the place of U12");
 
     const LuItem it = items[blockIdx.x];
-    const int n = it.n, m = lu_m(it), ncols = lu_ncols(it), kf = lu_kf(it), ntop = it.nt;
+    const int n = it.n, m = lu_m(it), kf = lu_kf(it), ntop = it.nt;
     if (k0 >= kf) return;
     const int ld = it.ld, tid = threadIdx.x, nth = blockDim.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rows = lu_rows(k0, m, ntop), kb = min(NB, kf - k0);
     const int panel = k0 / NB;
     double* re = it.re;
@@ -267,19 +315,41 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
 
     double ar[NB], ai[NB];
     int pos = tid;  // current position of this thread's original panel row
-    // full panels of 16-byte aligned rows move in 16-byte pieces (uniform over the workgroup)
+    // full panels of 16-byte aligned rows move in 16-byte pieces, eight lanes to a row's 128 bytes,
+    // and turn through LDS (uniform over the workgroup; a row per lane straight from memory takes a
+    // memory line per lane: 14200 and 9400 cycles for the loads and stores of 288 rows, now 8000
+    // and 7200)
     const bool vec = kb == NB && ld % 2 == 0 && ((reinterpret_cast<uintptr_t>(re) | reinterpret_cast<uintptr_t>(im)) & 15) == 0;
+    double* tr = big + wave * 64 * LU_TROW;
+    const int qrow = lane >> 3, qc = 2 * (lane & 7);  // this lane's row of eight and column pair in an access
     if (vec) {
-        const long o = own ? (long)lu_row(k0, ntop, tid) * ld + k0 : 0;
+        double2 v[2][NB / LU_TC][8];
 #pragma unroll
-        for (int c = 0; c < NB; c += 2) {
-            const double2 vr = own ? *reinterpret_cast<const double2*>(re + o + c) : make_double2(0.0, 0.0);
-            const double2 vi = own ? *reinterpret_cast<const double2*>(im + o + c) : make_double2(0.0, 0.0);
-            ar[c] = vr.x;
-            ar[c + 1] = vr.y;
-            ai[c] = vi.x;
-            ai[c + 1] = vi.y;
-        }
+        for (int h = 0; h < NB / LU_TC; ++h)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int t = wave * 64 + 8 * e + qrow;
+                const long o = t < rows ? (long)lu_row(k0, ntop, t) * ld + k0 + h * LU_TC + qc : 0;
+                v[0][h][e] = ld_global2(re + o);
+                v[1][h][e] = ld_global2(im + o);
+            }
+#pragma unroll
+        for (int h = 0; h < NB / LU_TC; ++h)
+#pragma unroll
+            for (int pl = 0; pl < 2; ++pl) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    *reinterpret_cast<double2*>(tr + (8 * e + qrow) * LU_TROW + qc) = v[pl][h][e];
+                lu_wave_lds();
+#pragma unroll
+                for (int c = 0; c < LU_TC; c += 2) {
+                    const double2 x = *reinterpret_cast<const double2*>(tr + lane * LU_TROW + c);
+                    double* d = (pl ? ai : ar) + h * LU_TC + c;
+                    d[0] = own ? x.x : 0.0;
+                    d[1] = own ? x.y : 0.0;
+                }
+                lu_wave_lds();
+            }
         if (add_identity && own && tid < NB) {
 #pragma unroll
             for (int c = 0; c < NB; ++c)
@@ -299,22 +369,28 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
         }
     }
 
-    __syncthreads();
     // Column loop.  Rows never move between threads: thread t keeps original panel row t in
     // registers and `pos` is its current position (LAPACK's interchange of rows KK and p is
-    // the exchange of two positions).  Columns go in groups of LU_CG: in the group starting at
-    // column K2 slot Q (0 .. LU_CG-1) holds column K2 + Q, and after the group the register
-    // row is rotated by LU_CG slots, the freed slots taking their columns' multipliers (rows
-    // still to be pivoted) or departing values (rows already pivoted).  After NB / LU_CG
+    // the exchange of two positions).  Columns go in groups of CG: in the group starting at
+    // column K2 slot Q (0 .. CG-1) holds column K2 + Q, and after the group the register
+    // row is rotated by CG slots, the freed slots taking their columns' multipliers (rows
+    // still to be pivoted) or departing values (rows already pivoted).  After NB / CG
     // rotations every row is back in column order, L multipliers then U entries.  This keeps
     // all register indices static inside a real loop (a fully unrolled column loop does not
-    // fit the instruction cache) at 1 / LU_CG of the register moves of a rotation per column.
-    constexpr int LU_CG = 8;
-    static_assert(NB % LU_CG == 0, "columns go in groups");
-    for (int k2 = 0; k2 < NB; k2 += LU_CG) {
-        const int live = NB - k2;  // slots Q+1 .. live-1 hold the columns right of column K2 + Q
+    // fit the instruction cache) at 1 / CG of the register moves of a rotation per column.
+    //
+    // A column step is one wave's chain of latencies (pivot search, two barriers, a reciprocal, the
+    // update), so it moves as little as it can: the pivot row's part in the group's own columns
+    // (grow) and their update.  The columns right of the group take all CG pivots at its end, from
+    // U12 = L11^{-1} A12 of the pivot rows (gu12), broadcast by DPP from one LDS read per 16 columns.
+    // One LU of order 288 averages 45 us a panel (53.6 us with every pivot updating all columns right
+    // of it and the rows straight from memory; 54.8 us with every wave posting its best candidate's
+    // row before a single barrier); order 128, 44 us a panel (49.7).
+    __syncthreads();
+    for (int k2 = 0; k2 < NB; k2 += CG) {
+        const int live = NB - k2;  // slots CG .. live-1 hold the columns right of the group
 #pragma unroll
-        for (int Q = 0; Q < LU_CG; ++Q) {
+        for (int Q = 0; Q < CG; ++Q) {
             const int kk = k2 + Q;
             double nr = ar[Q], ni = ai[Q];  // stays in slot Q: the multiplier or the departing value
             if (kk < kb) {
@@ -327,10 +403,9 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
                 // pivot position; an exactly zero column (no nonzero key) keeps row kk in place
                 const unsigned long long kmax = pkey[kk];
                 const int p = kmax ? 511 - static_cast<int>(kmax & 0x1FFull) : kk;
-                if (own && pos == p) {  // the raw register row (see the update for the other slots)
-                    double2* dst = reinterpret_cast<double2*>(xrow);
+                if (own && pos == p) {
 #pragma unroll
-                    for (int j = 0; j < NB; ++j) dst[j] = make_double2(ar[j], ai[j]);
+                    for (int j = 0; j < CG; ++j) grow[Q][j] = make_double2(ar[j], ai[j]);
                 }
                 if (own) {  // the interchange of positions kk and p
                     if (pos == p)
@@ -341,9 +416,10 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
                 if (tid == 0) pvt[kk] = p;  // global stores here would stall every LDS wait (FLAT)
                 __syncthreads();
                 if (own && pos > kk) {  // rows not yet pivoted: multiplier and rank-1 update
-                    const double2* xv = reinterpret_cast<const double2*>(xrow);
-                    const double2 u0 = xv[Q];
-                    const double ur = u0.x, ui = u0.y;
+                    double2 bv[CG];
+#pragma unroll
+                    for (int j = Q; j < CG; ++j) bv[j] = grow[Q][j];
+                    const double ur = bv[Q].x, ui = bv[Q].y;
                     if (ur != 0.0 || ui != 0.0) {
                         const double rden = 1.0 / (ur * ur + ui * ui);
                         const double ir = ur * rden, ii = -ui * rden;
@@ -351,92 +427,150 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
                         ni = nr * ii + ni * ir;
                         nr = t;
                     }
-                    // the pivot row in batches of 8 entries (a batch's reads in flight together).
-                    // Slots 0..Q and live.. of the pivot row hold its own multipliers (or, for
-                    // slots below Q, entries of columns already done): batches
-                    // from live on are skipped and the one batch that straddles live is masked
-                    // (the owner writes its row unmasked, a single lane's stores on the critical
-                    // path).  Two fused multiply-adds per real part:
-                    // a_j - m b_j = (a_j - m_r b_r) + m_i b_i, likewise for the imaginary part.
-                    constexpr int RB = 8;
+                    // a_j - m b_j = (a_j - m_r b_r) + m_i b_i, likewise for the imaginary part
 #pragma unroll
-                    for (int j0 = 0; j0 < NB; j0 += RB) {
-                        if (j0 < live) {
-                            double2 bv[RB];
-#pragma unroll
-                            for (int q = 0; q < RB; ++q) bv[q] = xv[j0 + q];
-                            if (j0 + RB <= live) {
-#pragma unroll
-                                for (int q = 0; q < RB; ++q) {
-                                    const int j = j0 + q;
-                                    if (j > Q) {
-                                        ar[j] = fma(ni, bv[q].y, fma(-nr, bv[q].x, ar[j]));
-                                        ai[j] = fma(-ni, bv[q].x, fma(-nr, bv[q].y, ai[j]));
-                                    }
-                                }
-                            } else {
-#pragma unroll
-                                for (int q = 0; q < RB; ++q) {
-                                    const int j = j0 + q;
-                                    if (j > Q && j < live) {
-                                        ar[j] = fma(ni, bv[q].y, fma(-nr, bv[q].x, ar[j]));
-                                        ai[j] = fma(-ni, bv[q].x, fma(-nr, bv[q].y, ai[j]));
-                                    }
-                                }
-                            }
-                        }
+                    for (int j = Q + 1; j < CG; ++j) {
+                        ar[j] = fma(ni, bv[j].y, fma(-nr, bv[j].x, ar[j]));
+                        ai[j] = fma(-ni, bv[j].x, fma(-nr, bv[j].y, ai[j]));
                     }
                 }
             }
             ar[Q] = nr;
             ai[Q] = ni;
         }
-        double hr[LU_CG], hi[LU_CG];
+        if (k2 + CG < kb) {  // columns right of the group: U12 of its pivot rows, then their update
+            const int gp = pos - k2;  // this row's place among the group's pivots
+            const bool piv_row = own && gp >= 0 && gp < CG;
+            if (piv_row) {
 #pragma unroll
-        for (int q = 0; q < LU_CG; ++q) {
+                for (int j = CG; j < NB; ++j)
+                    if (j < live) gu12[gp][j - CG] = make_double2(ar[j], ai[j]);
+            }
+            __syncthreads();
+            if (tid < live - CG) {  // one column per thread: rows in order, u_p -= l_pq u_q
+                double2 u[CG];
+#pragma unroll
+                for (int q = 0; q < CG; ++q) u[q] = gu12[q][tid];
+#pragma unroll
+                for (int q = 0; q < CG - 1; ++q)
+#pragma unroll
+                    for (int p = q + 1; p < CG; ++p) {
+                        const double2 l = grow[p][q];
+                        u[p].x = fma(l.y, u[q].y, fma(-l.x, u[q].x, u[p].x));
+                        u[p].y = fma(-l.y, u[q].x, fma(-l.x, u[q].y, u[p].y));
+                    }
+#pragma unroll
+                for (int q = 1; q < CG; ++q) gu12[q][tid] = u[q];
+            }
+            __syncthreads();
+            {  // every lane takes part (DPP); rows at or above the group with multiplier zero
+                const bool act = own && gp >= CG;
+                const int b0 = lane & 15, b1 = min(16 + (lane & 7), live - CG - 1);
+#pragma unroll
+                for (int q = 0; q < CG; ++q) {
+                    const double mr = act ? ar[q] : 0.0, mi = act ? ai[q] : 0.0;
+                    const double nmr = -mr, nmi = -mi;
+                    const double2 x = gu12[q][min(b0, live - CG - 1)];
+                    bcast_fma8<0>(ar + CG, ai + CG, x.x, x.y, nmr, mi, nmi);
+                    if (live > 2 * CG) bcast_fma8<8>(ar + 2 * CG, ai + 2 * CG, x.x, x.y, nmr, mi, nmi);
+                    if (live > 3 * CG) {
+                        const double2 y = gu12[q][b1];
+                        bcast_fma8<0>(ar + 3 * CG, ai + 3 * CG, y.x, y.y, nmr, mi, nmi);
+                    }
+                }
+            }
+            if (piv_row) {
+#pragma unroll
+                for (int j = CG; j < NB; ++j)
+                    if (j < live) {
+                        const double2 v = gu12[gp][j - CG];
+                        ar[j] = v.x;
+                        ai[j] = v.y;
+                    }
+            }
+        }
+        double hr[CG], hi[CG];
+#pragma unroll
+        for (int q = 0; q < CG; ++q) {
             hr[q] = ar[q];
             hi[q] = ai[q];
         }
 #pragma unroll
-        for (int j = 0; j < NB - LU_CG; ++j) {
-            ar[j] = ar[j + LU_CG];
-            ai[j] = ai[j + LU_CG];
+        for (int j = 0; j < NB - CG; ++j) {
+            ar[j] = ar[j + CG];
+            ai[j] = ai[j + CG];
         }
 #pragma unroll
-        for (int q = 0; q < LU_CG; ++q) {
-            ar[NB - LU_CG + q] = hr[q];
-            ai[NB - LU_CG + q] = hi[q];
+        for (int q = 0; q < CG; ++q) {
+            ar[NB - CG + q] = hr[q];
+            ai[NB - CG + q] = hi[q];
         }
     }
+    __syncthreads();  // pvt
     if (tid < kb) it.piv[k0 + tid] = lu_row(k0, ntop, pvt[tid]);
-    if (own) {
-        const long orow = lu_row(k0, ntop, pos);
-        if (vec) {
-#pragma unroll
-            for (int c = 0; c < NB; c += 2) {
-                *reinterpret_cast<double2*>(re + orow * ld + k0 + c) = make_double2(ar[c], ar[c + 1]);
-                *reinterpret_cast<double2*>(im + orow * ld + k0 + c) = make_double2(ai[c], ai[c + 1]);
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < NB; ++c) {
-                if (c < kb) {
-                    re[orow * ld + k0 + c] = ar[c];
-                    im[orow * ld + k0 + c] = ai[c];
-                }
-            }
+    if (own && pos != tid) {  // at most 2*NB positions change: the panel rows and their partners
+        const int sl = atomicAdd(&slot_cnt, 1);
+        if (sl < 2 * NB) {
+            slot_dst[sl] = pos;
+            slot_src[sl] = tid;
         }
-        if (pos != tid) {  // at most 2*NB positions change: the panel rows and their partners
-            const int sl = atomicAdd(&slot_cnt, 1);
-            if (sl < 2 * NB) {
-                slot_dst[sl] = pos;
-                slot_src[sl] = tid;
+    }
+    if (vec) {
+        drow[tid] = lu_row(k0, ntop, pos);
+        lu_wave_lds();
+        int orow[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) orow[e] = drow[wave * 64 + 8 * e + qrow];
+#pragma unroll
+        for (int h = 0; h < NB / LU_TC; ++h)
+#pragma unroll
+            for (int pl = 0; pl < 2; ++pl) {
+#pragma unroll
+                for (int c = 0; c < LU_TC; c += 2) {
+                    const double* d = (pl ? ai : ar) + h * LU_TC + c;
+                    *reinterpret_cast<double2*>(tr + lane * LU_TROW + c) = make_double2(d[0], d[1]);
+                }
+                lu_wave_lds();
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const double2 x = *reinterpret_cast<const double2*>(tr + (8 * e + qrow) * LU_TROW + qc);
+                    if (wave * 64 + 8 * e + qrow < rows)
+                        st_global2((pl ? im : re) + (long)orow[e] * ld + k0 + h * LU_TC + qc, x);
+                }
+                lu_wave_lds();
+            }
+    } else if (own) {
+        const long orow = lu_row(k0, ntop, pos);
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+            if (c < kb) {
+                re[orow * ld + k0 + c] = ar[c];
+                im[orow * ld + k0 + c] = ai[c];
             }
         }
     }
+    __syncthreads();  // the transposes are done with `big`
+    double(*lt_re)[NB + 1] = reinterpret_cast<double(*)[NB + 1]>(big);  // L11, inverted in place
+    double(*lt_im)[NB + 1] = lt_re + NB;
+    double(*ut_re)[NB + 1] = lt_im + NB;                                // U11, inverted in place
+    double(*ut_im)[NB + 1] = ut_re + NB;
+    double(*tl_re)[NB + 1] = ut_im + NB;                                // doubling temporaries
+    double(*tl_im)[NB + 1] = tl_re + NB;
+    double(*tu_re)[NB + 1] = tl_im + NB;
+    double(*tu_im)[NB + 1] = tu_re + NB;
     // L11 and U11 (diagonal inverted) into LDS from the rows now at positions 0..kb-1;
     // positions kb..NB-1 of a partial last panel are padded with the identity
-    if ((own && pos < NB) || (!own && tid < NB)) {
+    if (vec) {  // the rows just stored, read back coalesced (a full panel: no padding)
+        for (int e = tid; e < NB * NB; e += nth) {
+            const int r = e / NB, c = e % NB;
+            const long o = (long)lu_row(k0, ntop, r) * ld + k0 + c;
+            const double vr = re[o], vi = im[o];
+            lt_re[r][c] = c < r ? vr : (c == r ? 1.0 : 0.0);
+            lt_im[r][c] = c < r ? vi : 0.0;
+            ut_re[r][c] = c >= r ? vr : 0.0;
+            ut_im[r][c] = c >= r ? vi : 0.0;
+        }
+    } else if ((own && pos < NB) || (!own && tid < NB)) {
         const int r = own ? pos : tid;
         const bool in = own;
 #pragma unroll
