@@ -8,16 +8,18 @@
 // with the imaginary part reduced by the IEEE remainder to [-pi, pi]
 // (src/isle/cpp/math.hpp:265-293).
 //
-// The factorisation is right-looking in panels of LU_NB columns, two launches per panel:
-//   lu_panel_kernel  (one workgroup per matrix, one matrix row per thread, held in
-//                     registers): pivoted factorisation of the panel, L11^{-1} by
-//                     recursive doubling, the panel's interchanges on the columns right
-//                     of the panel (the new A12 rows are staged in the work buffer, the
-//                     displaced rows written in place), and on the item's last panel
-//                     the log-determinant;
-//   lu_update_kernel (32x32 tiles, every CU): U12 = L11^{-1} A12 and
-//                     A22 -= L21 U12 on FP64 MFMA, plus the panel's interchanges on the
-//                     columns left of it.
+// The factorisation is right-looking in panels of LU_NB columns, one launch per panel and one at the end:
+//   lu_step_kernel   one workgroup per matrix (the chain that the whole factorisation waits for) first
+//                    takes the elimination of the panel before on the next panel's own columns, then
+//                    factorises that panel (one matrix row per thread, held in registers) with its
+//                    L11^{-1} and U11^{-1} and, on the item's last panel, the log-determinant; beside it
+//                    one workgroup per strip of LU_NB further columns takes the elimination of the panel
+//                    before there (interchanges, U12 = L11^{-1} A12, A22 -= L21 U12 on FP64 MFMA), and
+//                    more take its interchanges on the columns that are finished or not eliminated.
+// Against a launch each for the panel, the interchanges and tiles of the elimination: order 288,
+// 704 -> 555 us for 32 matrices, 560 -> 526 us for one; order 128, 250 -> 213 us for 32.  Panels of more than LU_MAX_N candidate rows are factorised in global
+// memory (lu_panel_tall_kernel) and keep those launches (lu_rswap_kernel, lu_update_kernel): a strip of
+// so many rows is too much work for one workgroup, and few strips would leave CUs idle.
 //
 // Besides square matrices the same kernels factorise the first kf columns of an m x ncols
 // matrix whose rows [k0+NB, nt) are, in the columns not yet factorised, known to be rows of
@@ -66,13 +68,14 @@ __host__ __device__ inline int lu_row(int k0, int nt, int p) {
 
 // Work layout: for every panel p, L11^{-1} and U11^{-1} of that panel ([NB][NB] re and im
 // planes each; a partial last panel is padded with the identity), then the staged A12
-// rows [NB][n] re and im planes, then the panel's composed interchange as ints
-// {count, dst[2NB], src[2NB]}.  The diagonal-block inverses stay valid after the
-// factorisation and are used by the triangular solve.
+// rows [NB][n] re and im planes (only for panels taller than LU_MAX_N), then the composed interchanges
+// of the panel and of the one before it (by parity) as ints {count, dst[2NB], src[2NB]}.  The
+// diagonal-block inverses stay valid after the factorisation and are used by the triangular solve.
 constexpr int LU_DINV = 4 * LU_NB * LU_NB;  // doubles per panel: L11^{-1}, U11^{-1} (re, im)
+constexpr int LU_PERM = 2 * LU_NB + 2;      // doubles per interchange record
 __host__ __device__ inline int lu_panels(int n) { return (n + LU_NB - 1) / LU_NB; }
 __host__ __device__ inline size_t lu_work_doubles(int kf, int ncols) {
-    return (size_t)LU_DINV * lu_panels(kf) + 2 * (size_t)LU_NB * ncols + 2 * LU_NB + 2;
+    return (size_t)LU_DINV * lu_panels(kf) + 2 * (size_t)LU_NB * ncols + 2 * LU_PERM;
 }
 __host__ __device__ inline size_t lu_work_doubles(int n) { return lu_work_doubles(n, n); }
 __device__ inline double* lu_linv(const LuItem& it, int panel) { return it.work + (size_t)LU_DINV * panel; }
@@ -80,8 +83,8 @@ __device__ inline double* lu_uinv(const LuItem& it, int panel) {
     return it.work + (size_t)LU_DINV * panel + 2 * LU_NB * LU_NB;
 }
 __device__ inline double* lu_stage(const LuItem& it) { return it.work + (size_t)LU_DINV * lu_panels(lu_kf(it)); }
-__device__ inline int* lu_perm(const LuItem& it) {
-    return reinterpret_cast<int*>(lu_stage(it) + 2 * (size_t)LU_NB * lu_ncols(it));
+__device__ inline int* lu_perm(const LuItem& it, int panel) {
+    return reinterpret_cast<int*>(lu_stage(it) + 2 * (size_t)LU_NB * lu_ncols(it) + (panel & 1) * LU_PERM);
 }
 
 __device__ __forceinline__ double cabs1(double r, double i) { return fabs(r) + fabs(i); }
@@ -160,7 +163,10 @@ __device__ __forceinline__ void bcast_fma8(double* ar, double* ai, double br, do
     bcast_fma4<J0 + 4>(ar + 4, ai + 4, br, bi, nmr, mi, nmi);
 }
 
-// 16-byte global accesses, and a wave's own LDS traffic in order (one wave writes and reads: no barrier)
+// 8- and 16-byte global accesses, and a wave's own LDS traffic in order (one wave writes and reads: no barrier)
+__device__ __forceinline__ double ld_global1(const double* p) {
+    return *(__attribute__((address_space(1))) const double*)p;
+}
 __device__ __forceinline__ double2 ld_global2(const double* p) {
     typedef double dbl2 __attribute__((ext_vector_type(2)));
     const dbl2 v = *(__attribute__((address_space(1))) const dbl2*)p;
@@ -273,13 +279,185 @@ __device__ inline void lu_panel_logdet(const LuItem& it, int k0, int nb, int kf,
     }
 }
 
+// The interchanges of the panel at kp on columns [c0, c1) (at most LU_SWAP_COLS): every displaced row is
+// read before any is written.  All threads of the workgroup (at least LU_UPD_THREADS).
+__device__ inline void lu_swap_columns(const LuItem& it, int kp, int c0, int c1) {
+    constexpr int PER = 2 * LU_NB * LU_SWAP_COLS / LU_UPD_THREADS;
+    const int tid = threadIdx.x, nth = blockDim.x, ntop = it.nt, ld = it.ld;
+    const int* perm = lu_perm(it, kp / LU_NB);
+    const int cnt = min(perm[0], 2 * LU_NB);
+    double vr[PER], vi[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int e = tid + j * nth, q = e / LU_SWAP_COLS, c = c0 + e % LU_SWAP_COLS;
+        if (q < cnt && c < c1) {
+            const long o = (long)lu_row(kp, ntop, perm[1 + 2 * LU_NB + q]) * ld + c;
+            vr[j] = it.re[o];
+            vi[j] = it.im[o];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int e = tid + j * nth, q = e / LU_SWAP_COLS, c = c0 + e % LU_SWAP_COLS;
+        if (q < cnt && c < c1) {
+            const long o = (long)lu_row(kp, ntop, perm[1 + q]) * ld + c;
+            it.re[o] = vr[j];
+            it.im[o] = vi[j];
+        }
+    }
+}
+
+// The elimination of the panel at kp on the LU_NB columns from c0 on (up to column nupd), by one
+// workgroup of at least four waves: the interchanges, U12 = L11^{-1} A12 and A22 -= L21 U12, in place.
+// One workgroup owns the strip, so the interchanged rows need no staging: from[p] is the position whose
+// old row the panel position p takes, every read of an old panel row comes before U12 goes there, and a
+// position below the panel takes either its own row or an old panel row.
+// MFMA operands come straight from memory (four consecutive k per instruction, in order, as
+// lu_update_kernel); U12 stays in registers for all row tiles of a wave.
+constexpr int LU_SROW = LU_NB + 16;                      // 16 lanes each of two rows on all LDS banks
+constexpr int LU_STRIP_LDS = 2 * LU_NB * LU_SROW;        // doubles: U12
+__device__ inline void lu_strip_update(const LuItem& it, int kp, int c0, double* su, unsigned short* from) {
+    constexpr int NB = LU_NB;
+    const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6;
+    const int li = lane & 15, lk = lane >> 4;
+    const int ld = it.ld, ntop = it.nt, rows = lu_rows(kp, lu_m(it), ntop), c1 = lu_nupd(it);
+    const int below = lu_structured(kp, ntop) ? ntop - NB : kp;  // matrix row of position p >= NB, minus p
+    const int prow = min(NB, rows);
+    double* re = it.re;
+    double* im = it.im;
+    double* su_re = su;
+    double* su_im = su + NB * LU_SROW;
+    const int* perm = lu_perm(it, kp / NB);
+    const int cnt = min(perm[0], 2 * NB);
+    int pd = 0, ps = 0;
+    if (tid < cnt) {
+        pd = perm[1 + tid];
+        ps = perm[1 + 2 * NB + tid];
+    }
+    for (int p = tid; p < max(rows, NB); p += nth) from[p] = (unsigned short)p;
+    __syncthreads();
+    if (tid < cnt) from[pd] = (unsigned short)ps;
+    __syncthreads();
+    auto row_of = [&](int f) { return f < NB ? kp + f : below + f; };
+
+    // row tile t: 16 positions from NB + 16 t; L21 rows and the strip's entries
+    const int tiles = (rows - NB + 15) / 16;  // <= 0 when there is nothing below
+    struct Tile {
+        double lr[8], li[8], cr[2][4], ci[2][4];
+    };
+    auto load = [&](Tile& x, int t) {
+        const int p = NB + 16 * t + li;
+        const long o = (long)(below + min(p, rows - 1)) * ld + kp + lk;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            x.lr[e] = ld_global1(re + o + 4 * e);
+            x.li[e] = ld_global1(im + o + 4 * e);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const long oc = (long)row_of(from[min(NB + 16 * t + lk + 4 * r, rows - 1)]) * ld;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int c = min(c0 + 16 * h + li, c1 - 1);
+                x.cr[h][r] = ld_global1(re + oc + c);
+                x.ci[h][r] = ld_global1(im + oc + c);
+            }
+        }
+    };
+    Tile x;
+    if (wave < tiles) load(x, wave);
+    if (wave < 4) {  // U12 tile of this wave
+        const int wm = (wave >> 1) * 16, wn = (wave & 1) * 16, c = c0 + wn + li;
+        const double* linv = lu_linv(it, kp / NB) + (wm + li) * NB + lk;
+        dbl4 rr = {0, 0, 0, 0}, ii = rr, ri = rr, ir = rr;
+        double a_r[8], a_i[8], b_r[8], b_i[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            a_r[e] = ld_global1(linv + 4 * e);
+            a_i[e] = ld_global1(linv + NB * NB + 4 * e);
+            const int q = 4 * e + lk;
+            const bool in = q < prow && c < c1;
+            const long o = in ? (long)row_of(from[q]) * ld + c : 0;
+            b_r[e] = ld_global1(re + o);
+            b_i[e] = ld_global1(im + o);
+            b_r[e] = in ? b_r[e] : 0.0;
+            b_i[e] = in ? b_i[e] : 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            rr = mfma16(a_r[e], b_r[e], rr);
+            ii = mfma16(a_i[e], b_i[e], ii);
+            ri = mfma16(a_r[e], b_i[e], ri);
+            ir = mfma16(a_i[e], b_r[e], ir);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            su_re[(wm + lk + 4 * r) * LU_SROW + wn + li] = rr[r] - ii[r];
+            su_im[(wm + lk + 4 * r) * LU_SROW + wn + li] = ri[r] + ir[r];
+        }
+    }
+    __syncthreads();
+    if (wave < tiles) {
+        double u_r[2][8], u_i[2][8];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                u_r[h][e] = su_re[(4 * e + lk) * LU_SROW + 16 * h + li];
+                u_i[h][e] = su_im[(4 * e + lk) * LU_SROW + 16 * h + li];
+            }
+        for (int t = wave; t < tiles; t += nw) {
+            Tile y = x;
+            if (t + nw < tiles) load(x, t + nw);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                dbl4 rr = {0, 0, 0, 0}, ii = rr, ri = rr, ir = rr;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    rr = mfma16(y.lr[e], u_r[h][e], rr);
+                    ii = mfma16(y.li[e], u_i[h][e], ii);
+                    ri = mfma16(y.lr[e], u_i[h][e], ri);
+                    ir = mfma16(y.li[e], u_r[h][e], ir);
+                }
+                const int c = c0 + 16 * h + li;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int p = NB + 16 * t + lk + 4 * r;
+                    if (p < rows && c < c1) {
+                        const long o = (long)(below + p) * ld + c;
+                        re[o] = y.cr[h][r] - (rr[r] - ii[r]);
+                        im[o] = y.ci[h][r] - (ri[r] + ir[r]);
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();  // every old panel row has been read
+    for (int e = tid; e < NB * NB; e += nth) {
+        const int q = e / NB, c = e % NB;
+        if (q < prow && c0 + c < c1) {
+            re[(long)(kp + q) * ld + c0 + c] = su_re[q * LU_SROW + c];
+            im[(long)(kp + q) * ld + c0 + c] = su_im[q * LU_SROW + c];
+        }
+    }
+    __syncthreads();
+}
+
 // Rows of a wave between row-per-lane registers and coalesced memory accesses: a wave's 64 rows of
 // LU_TC columns of one plane in LDS, padded to 16 bytes off a power of two.
 constexpr int LU_TC = 16, LU_TROW = LU_TC + 2;
 
+// One step of the factorisation: the panel at k0 (-1: none) of every item, and the elimination of the panel
+// at kp (-1: none) on the columns from cs on.  grid.x: nitems panel workgroups if k0 >= 0, then for each
+// unit one workgroup per item: `strips` of LU_NB columns, `defer` of LU_SWAP_COLS columns that take the
+// interchanges only, then the columns left of kp.  Items vary fastest, so the units of an item run on
+// its panel's XCD (L21 and the record come from its L2) when their number is a multiple of 8.  The
+// workgroups of one launch write disjoint columns and read, besides their own, only those of panel kp.
 template <int NB>
-__global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __restrict__ items, int k0,
-                                                            int add_identity) {
+__global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restrict__ items, int nitems, int k0,
+                                                           int add_identity, int kp, int cs, int strips, int defer) {
     constexpr int CG = 8, MAXW = LU_MAX_N / 64;  // columns per group, waves
     static_assert(NB % LU_TC == 0 && NB % CG == 0, "columns go in groups");
     constexpr int TRI = NB * (NB + 1);           // one NB x (NB + 1) plane
@@ -297,9 +475,28 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
     int* drow = reinterpret_cast<int*>(&gu12[0][0]);
     static_assert(sizeof(gu12) >= LU_MAX_N * sizeof(int), "row numbers in the place of U12");
 
-    const LuItem it = items[blockIdx.x];
+    // `big` before the panel's own rows: U12 of the panel at kp and its row positions
+    unsigned short* from = reinterpret_cast<unsigned short*>(big + LU_STRIP_LDS);
+    static_assert(sizeof(big) >= LU_STRIP_LDS * sizeof(double) + LU_MAX_N * sizeof(unsigned short), "strip in LDS");
+    const int item = blockIdx.x % nitems, unit = blockIdx.x / nitems - (k0 >= 0 ? 1 : 0);
+    const LuItem it = items[item];
     const int n = it.n, m = lu_m(it), kf = lu_kf(it), ntop = it.nt;
+    if (unit >= 0) {  // the panel at kp on the other columns (uniform over the workgroup)
+        if (kp >= kf) return;
+        const int ce = lu_nupd(it), cd = max(cs, ce);  // columns cs .. ce take the elimination, cd .. the interchanges
+        if (unit < strips) {
+            if (cs + LU_NB * unit < ce) lu_strip_update(it, kp, cs + LU_NB * unit, big, from);
+        } else if (unit < strips + defer) {
+            const int c = cd + LU_SWAP_COLS * (unit - strips);
+            if (c < lu_ncols(it)) lu_swap_columns(it, kp, c, lu_ncols(it));
+        } else {
+            const int c = LU_SWAP_COLS * (unit - strips - defer);
+            if (c < kp) lu_swap_columns(it, kp, c, kp);
+        }
+        return;
+    }
     if (k0 >= kf) return;
+    if (kp >= 0) lu_strip_update(it, kp, k0, big, from);
     const int ld = it.ld, tid = threadIdx.x, nth = blockDim.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rows = lu_rows(k0, m, ntop), kb = min(NB, kf - k0);
@@ -590,7 +787,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
         ut_im[tid][tid] = -vi / den;
     }
     const int cnt = min(slot_cnt, 2 * NB);
-    int* perm = lu_perm(it);
+    int* perm = lu_perm(it, panel);
     for (int e = tid; e < cnt; e += nth) {
         perm[1 + e] = slot_dst[e];
         perm[1 + 2 * NB + e] = slot_src[e];
@@ -608,7 +805,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_panel_kernel(const LuItem* __rest
 // row.  Per column: pivot search (keys as in pivot_key, 14 position bits), the pivot row
 // swapped with row kk across the panel's columns and copied to LDS, then the multipliers
 // and the rank-1 update of the rows below.  The interchange record, L11^{-1} / U11^{-1} and
-// the log-determinant are those of lu_panel_kernel.
+// the log-determinant are those of lu_step_kernel.
 constexpr int LU_TALL_MAX = 16383;
 constexpr int LU_TALL_THREADS = 1024;
 
@@ -724,7 +921,7 @@ __global__ __launch_bounds__(LU_TALL_THREADS) void lu_panel_tall_kernel(const Lu
             org[a] = org[b];
             org[b] = t;
         }
-        int* perm = lu_perm(it);
+        int* perm = lu_perm(it, k0 / NB);
         int w = 0;
         for (int e = 0; e < cnt; ++e)
             if (org[e] != pos[e]) {
@@ -778,7 +975,7 @@ __global__ __launch_bounds__(256) void lu_rswap_kernel(const LuItem* __restrict_
     if (c0 >= nrt) return;
     __shared__ int orig[NB], dst[2 * NB], src[2 * NB];
     __shared__ int cnt_s;
-    const int* perm = lu_perm(it);
+    const int* perm = lu_perm(it, k0 / LU_NB);
     const int tid = threadIdx.x;
     if (tid == 0) cnt_s = min(perm[0], 2 * NB);
     if (tid < NB) orig[tid] = tid;
@@ -869,7 +1066,7 @@ __global__ __launch_bounds__(LU_UPD_THREADS) void lu_update_kernel(const LuItem*
         // ---- interchanges of this panel on LU_SWAP_COLS columns left of it
         const int c0 = ((int)blockIdx.x - tmr * tmc) * LU_SWAP_COLS;
         if (c0 >= k0) return;
-        const int* perm = lu_perm(it);
+        const int* perm = lu_perm(it, k0 / LU_NB);
         const int cnt = perm[0];
         constexpr int PER = 2 * NB * LU_SWAP_COLS / LU_UPD_THREADS;
         double vr[PER], vi[PER];
@@ -991,7 +1188,7 @@ __global__ __launch_bounds__(LU_UPD_THREADS) void lu_update_kernel(const LuItem*
 
 // Factorise the first kf columns of nitems m x ncols matrices of one shape (identity rows
 // above nt as described at the top; nt = 0 for a general matrix).  Panels with at most
-// LU_MAX_N candidate rows run in registers (lu_panel_kernel), larger ones up to LU_TALL_MAX
+// LU_MAX_N candidate rows run in registers (lu_step_kernel), larger ones up to LU_TALL_MAX
 // in global memory (lu_panel_tall_kernel).
 inline void launch_lu_shape(const LuItem* d_items, int nitems, int m, int ncols, int kf, int nt, int add_identity,
                             hipStream_t s, int nupd = 0) {
@@ -999,20 +1196,37 @@ inline void launch_lu_shape(const LuItem* d_items, int nitems, int m, int ncols,
         throw std::invalid_argument("inconsistent LU shape");
     for (int k0 = 0; k0 < kf; k0 += LU_NB)
         if (lu_rows(k0, m, nt) > LU_TALL_MAX) throw std::invalid_argument("matrix too large for the LU kernel");
+    if (nitems <= 0) return;
+    const int nu = nupd > 0 ? std::min(nupd, ncols) : ncols;
+    int kp = -1;  // the panel whose elimination is still to come, in registers so far (-1: none)
+    // the launch of the panel at k0 (-1: none) and of kp's elimination
+    auto step = [&](int k0) {
+        const int cs = k0 >= 0 ? k0 + LU_NB : kp + LU_NB;
+        const int strips = kp >= 0 ? std::max(0, nu - cs + LU_NB - 1) / LU_NB : 0;
+        const int cd = std::max(cs, nu), defer = kp >= 0 ? std::max(0, ncols - cd + LU_SWAP_COLS - 1) / LU_SWAP_COLS : 0;
+        const int left = kp >= 0 ? (kp + LU_SWAP_COLS - 1) / LU_SWAP_COLS : 0;
+        const int units = (k0 >= 0 ? 1 : 0) + strips + defer + left;
+        if (units == 0) return;
+        const int rows = lu_rows(kp >= 0 ? kp : k0, m, nt);
+        // at least 4 waves: the strips and the inversion of L11 and U11 take that many
+        const int threads = std::max(256, ((rows + 63) / 64) * 64);
+        hipLaunchKernelGGL(lu_step_kernel<LU_NB>, dim3(units * nitems), dim3(threads), 0, s, d_items, nitems, k0,
+                           k0 == 0 ? add_identity : 0, kp, cs, strips, defer);
+        ISLE_HIP(hipGetLastError());
+    };
     for (int k0 = 0; k0 < kf; k0 += LU_NB) {
         const int rows = lu_rows(k0, m, nt);
-        if (rows > LU_MAX_N) {  // the panel in global memory
-            hipLaunchKernelGGL(lu_panel_tall_kernel<LU_NB>, dim3(nitems), dim3(LU_TALL_THREADS), 0, s, d_items, k0,
-                               k0 == 0 ? add_identity : 0);
-        } else {
-            // at least 4 waves: the L11 / U11 inversion after the column loop uses every thread
-            const int threads = std::max(256, ((rows + 63) / 64) * 64);
-            hipLaunchKernelGGL(lu_panel_kernel<LU_NB>, dim3(nitems), dim3(threads), 0, s, d_items, k0,
-                               k0 == 0 ? add_identity : 0);
+        if (rows <= LU_MAX_N) {
+            step(k0);
+            kp = k0;
+            continue;
         }
+        // the panel in global memory, its elimination on tiles (rows do not grow with k0: none is pending)
+        hipLaunchKernelGGL(lu_panel_tall_kernel<LU_NB>, dim3(nitems), dim3(LU_TALL_THREADS), 0, s, d_items, k0,
+                           k0 == 0 ? add_identity : 0);
         ISLE_HIP(hipGetLastError());
         const int ntr = rows - LU_NB, nsw = ncols - k0 - LU_NB;  // columns right of the panel
-        const int ntc = (nupd > 0 ? std::min(nupd, ncols) : ncols) - k0 - LU_NB;  // of them updated
+        const int ntc = nu - k0 - LU_NB;                         // of them updated
         if (nsw > 0) {
             hipLaunchKernelGGL(lu_rswap_kernel, dim3((nsw + 63) / 64, nitems), dim3(256), 0, s, d_items, k0);
             ISLE_HIP(hipGetLastError());
@@ -1025,6 +1239,9 @@ inline void launch_lu_shape(const LuItem* d_items, int nitems, int m, int ncols,
                                d_items, k0, tmr, tmc);
             ISLE_HIP(hipGetLastError());
         }
+    }
+    if (kp >= 0) {  // the last panel's interchanges, and its elimination on columns beyond kf
+        step(-1);
     }
 }
 

@@ -3150,7 +3150,7 @@ static constexpr int NOALLOC_MAX_N = 512;
 static constexpr size_t noalloc_align(size_t b) { return (b + 255) & ~size_t(255); }
 static constexpr size_t NOALLOC_WORK =
     (size_t)isle::LU_DINV * ((NOALLOC_MAX_N + isle::LU_NB - 1) / isle::LU_NB) + 2 * (size_t)isle::LU_NB * NOALLOC_MAX_N +
-    2 * isle::LU_NB + 2;  // lu_work_doubles(NOALLOC_MAX_N)
+    2 * isle::LU_PERM;  // lu_work_doubles(NOALLOC_MAX_N)
 static constexpr size_t NOALLOC_OFF_W = noalloc_align(2 * sizeof(double) * NOALLOC_MAX_N * NOALLOC_MAX_N);
 static constexpr size_t NOALLOC_OFF_PIV = NOALLOC_OFF_W + noalloc_align(NOALLOC_WORK * sizeof(double));
 static constexpr size_t NOALLOC_OFF_ITEM = NOALLOC_OFF_PIV + noalloc_align(NOALLOC_MAX_N * sizeof(int));
