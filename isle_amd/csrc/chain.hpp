@@ -92,7 +92,8 @@ __global__ __launch_bounds__(256) void chain_pack_kernel(const double* __restric
 
 // Suffix chain of one group of slices:  S_f = D_f A, then S_t = D_t A S_{t - dir} for the slices
 // after f in direction dir (-1: from the group's last slice to its first).  pre: the phases on the
-// other side, S_f = A D_f, S_t = A D_t S_{t - dir}.
+// other side, S_f = A D_f, S_t = A D_t S_{t - dir}; stored transposed these are, A being symmetric,
+// the prefix products D_f A D_{f + dir} A ... D_t A.
 struct SuffixItem {
     const double* packed;       // A in chain_pack_kernel's order
     const double* a;            // A, n x n row-major
@@ -101,8 +102,9 @@ struct SuffixItem {
     double* out;                // S_f transposed: re plane, im plane n n after it; each next one at
     long step;                  // + step; the last one is stored as it is, not transposed
     int first, dir, count;      // slice f, -1 or +1, slices in the group
-    int all;                    // 1: store every S_t (not with pre); 0: store the last one only (at out)
+    int all;                    // 1: store every S_t; 0: store the last one only (at out)
     int pre;
+    int keep = 0;               // 1: the last one transposed like the others
 };
 
 // Right chain of one group:  R_s = K D_s A, R_t = R_{t-1} D_t A, and the force diagonal
@@ -348,8 +350,8 @@ void suffix_chain_kernel(const SuffixItem* __restrict__ items, int n, int ntiles
                     for (int r = 0; r < 4; ++r) {
                         double* o = out + (tile * 16 + 4 * r * n);
                         if (c0 + 4 * r + lk < n && j < n) {
-                            st_lane(o, off, vr[r]);
-                            st_lane(o + nn, off, vi[r]);
+                            st_lane(o, off, it.pre ? re[i][r] : vr[r]);
+                            st_lane(o + nn, off, it.pre ? im[i][r] : vi[r]);
                         }
                     }
                 }
@@ -358,8 +360,9 @@ void suffix_chain_kernel(const SuffixItem* __restrict__ items, int n, int ntiles
                 for (int r = 0; r < 4; ++r) {
                     const int c = c0 + 4 * r + lk;
                     if (c < n && j < n) {
-                        st_global(out + (long)j * n + c, vr[r]);
-                        st_global(out + nn + (long)j * n + c, vi[r]);
+                        const long o = it.keep ? (long)c * n + j : (long)j * n + c;
+                        st_global(out + o, vr[r]);
+                        st_global(out + nn + o, vi[r]);
                     }
                 }
             }

@@ -52,6 +52,7 @@ struct LuItem {
     int nt = 0;      // > 0: rows [k0 + LU_NB, nt) are identity rows, never candidates (see above)
     int nupd = 0;    // > 0: columns [nupd, ncols) take the row interchanges only (their
                      // elimination is left to the caller: U12 = L11^{-1} A12, A22 -= L21 U12)
+    int add = 0;     // 1: factorise 1 + A, as the launch's add_identity for this matrix alone
 };
 __host__ __device__ inline int lu_m(const LuItem& it) { return it.m ? it.m : it.n; }
 __host__ __device__ inline int lu_ncols(const LuItem& it) { return it.ncols ? it.ncols : it.n; }
@@ -506,6 +507,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
     const bool own = tid < rows;
     if (tid == 0) slot_cnt = 0;
     if (tid < NB) pkey[tid] = 0ull;
+    if (k0 == 0) add_identity |= it.add;
     if (add_identity) {
         for (int i = NB + tid; i < n; i += nth) re[(long)i * ld + i] += 1.0;
     }
@@ -834,6 +836,7 @@ __global__ __launch_bounds__(LU_TALL_THREADS) void lu_panel_tall_kernel(const Lu
     const int panel = k0 / NB;
     double* re = it.re;
     double* im = it.im;
+    if (k0 == 0) add_identity |= it.add;
     if (add_identity)
         for (int i = tid; i < n; i += nth) re[(long)i * ld + i] += 1.0;
     __syncthreads();
@@ -1269,6 +1272,7 @@ struct SolveItem {
     long xsr, xsc;
     int n, ld, nrhs;
     int mode = 7;
+    long xoff = 0;  // x_re null: X at the launch's x_base + xoff, interleaved
 };
 enum : int { SOLVE_PERM = 1, SOLVE_L = 2, SOLVE_U = 4 };
 
@@ -1289,12 +1293,17 @@ inline size_t lu_solve_lds(int n) {
 // LU_MAX_N), B and X may be the same array.  GX = true: X kept in the output array itself
 // (larger orders; only the row permutation in LDS), so B must be null or another array.
 template <bool GX>
-__global__ __launch_bounds__(SOLVE_THREADS) void lu_solve_kernel(const SolveItem* __restrict__ items) {
+__global__ __launch_bounds__(SOLVE_THREADS) void lu_solve_kernel(const SolveItem* __restrict__ items,
+                                                              double* x_base) {
     extern __shared__ double lds[];
     __shared__ double part_r[4][16][17], part_i[4][16][17];
     __shared__ double dg_r[16][17], dg_i[16][17];  // inverse of the diagonal block
     __shared__ double y_r[16][17], y_i[16][17];    // right-hand side of the diagonal block
-    const SolveItem it = items[blockIdx.y];
+    SolveItem it = items[blockIdx.y];
+    if (!it.x_re) {
+        it.x_re = x_base + it.xoff;
+        it.x_im = it.x_re + 1;
+    }
     const int n = it.n, ld = it.ld;
     const int c0 = blockIdx.x * SOLVE_COLS;
     if (c0 >= it.nrhs) return;
@@ -1439,19 +1448,20 @@ __global__ __launch_bounds__(SOLVE_THREADS) void lu_solve_kernel(const SolveItem
     }
 }
 
-inline void launch_lu_solve(const SolveItem* d_items, int nitems, int max_n, int max_rhs, hipStream_t s) {
+inline void launch_lu_solve(const SolveItem* d_items, int nitems, int max_n, int max_rhs, hipStream_t s,
+                            double* x_base = nullptr) {
     dim3 grid((max_rhs + SOLVE_COLS - 1) / SOLVE_COLS, nitems);
     const size_t lds = lu_solve_lds(max_n);
     if (max_n <= LU_MAX_N && lds <= 134 * 1024) {
         ISLE_HIP(hipFuncSetAttribute((const void*)lu_solve_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)lds));
-        hipLaunchKernelGGL(lu_solve_kernel<false>, grid, dim3(SOLVE_THREADS), lds, s, d_items);
+        hipLaunchKernelGGL(lu_solve_kernel<false>, grid, dim3(SOLVE_THREADS), lds, s, d_items, x_base);
     } else {
         if (max_n > LU_TALL_MAX) throw std::invalid_argument("matrix too large for the LU solve kernel");
         const size_t lds_gx = 2 * (size_t)max_n * sizeof(int);
         ISLE_HIP(hipFuncSetAttribute((const void*)lu_solve_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)lds_gx));
-        hipLaunchKernelGGL(lu_solve_kernel<true>, grid, dim3(SOLVE_THREADS), lds_gx, s, d_items);
+        hipLaunchKernelGGL(lu_solve_kernel<true>, grid, dim3(SOLVE_THREADS), lds_gx, s, d_items, x_base);
     }
     ISLE_HIP(hipGetLastError());
 }

@@ -552,6 +552,8 @@ void Plan::set_tile(int kind, int tile) {
     };
     for (auto& kv : cache_) apply(*kv.second);
     for (auto& kv : multi_) apply(kv.second->merged);
+    for (OpCache* op : {sf_.products[0].get(), sf_.products[1].get(), sf_.rhs.get(), sf_.last.get(), sf_.every.get()})
+        if (op) apply(*op);
 }
 
 static bool is_gemm(K k) {
@@ -2561,87 +2563,115 @@ double* Plan::solve_workspace(size_t doubles) {
     return solve_ws_->as<double>();
 }
 
-// solveM (hubbardFermiMatrixExp.cpp:645-694, hubbardFermiMatrixDia.cpp:617-673).
-void Plan::solveM(const double* phi, int nt, int species, const double* rhss, int nrhs, double* out, bool reuse) {
+// Products, LUs and launch descriptors that solveM keeps between calls (sf_), for nt slices; reuse: the
+// factorisation of the last call is still wanted.  Everything is made once per nt, the descriptors per
+// species.
+void Plan::solve_factor(const double* phi, int nt, int species) {
     const int n = nx_;
     const long nn = (long)n * n;
     hipStream_t s = stream_;
-    const bool refactor = !(reuse && sf_.nt == nt && sf_.species == species && sf_.part);
-    if (refactor) {
+    if (sf_.nt != nt) {
         sf_ = SolveFactor{};
         sf_.ph.reset(new DevBuf((size_t)2 * nt * n * sizeof(double)));
         sf_.part.reset(new DevBuf((size_t)nt * 2 * nn * sizeof(double)));
         sf_.mz.reset(new DevBuf((size_t)nt * 2 * nn * sizeof(double)));
         sf_.piv.reset(new DevBuf((size_t)nt * n * sizeof(int)));
         sf_.luw.reset(new DevBuf((size_t)nt * lu_work_doubles(n) * sizeof(double)));
+        sf_.nt = nt;
     }
+    sf_.species = -1;
     double* ph = sf_.ph->as<double>();
     double* part = sf_.part->as<double>();
-    double* Mz = sf_.mz->as<double>();  // matrices multiplying the rhs (EXP: a copy of the partial products)
-    int* piv = sf_.piv->as<int>();
-    double* luw_p = sf_.luw->as<double>();
-    // right-hand-side buffers: Bt, Z (nt blocks of 2 n nrhs), Xl and a scratch block
-    const size_t rblk = (size_t)2 * n * nrhs;
-    double* Bt = solve_workspace((2 * (size_t)nt + 2) * rblk);
-    double* Z = Bt + (size_t)nt * rblk;
-    double* Xl = Z + (size_t)nt * rblk;
-    double* Sc = Xl + rblk;
+    double* Mz = sf_.mz->as<double>();
     auto D = [&](int t) { return CMat<double>{ph + (long)t * n, ph + (long)nt * n + (long)t * n}; };
     auto mP = [&](int t) { return cmat(part, t, nn); };
     auto mM = [&](int t) { return cmat(Mz, t, nn); };
-    if (refactor) {
-        OpCache op;
-        op.nt = nt;
-        op.phi_stride = 0;
-        Builder b(op);
+    if (!sf_.products[species]) {
+        std::unique_ptr<OpCache> op(new OpCache);
+        op->nt = nt;
+        op->phi_stride = 0;
+        Builder b(*op);
         std::vector<PhaseItem> phs{{0, 0, sigma_of(species), D(0).re, D(0).im, nullptr, nullptr, n, nt}};
         b.add(K::PHASE, phs);
         const double* A = a64_[species]->as<double>();
-        std::vector<ScaleItem<double>> sc{{A, D(0).re, D(0).im, mP(0).re, mP(0).im, n, SCALE_ROW}};
+        std::vector<ScaleItem<double>> sc;
         if (hop_ == DIA) sc.push_back({ident64_->as<double>(), D(0).re, D(0).im, mM(0).re, mM(0).im, n, SCALE_ROW});
-        b.add(K::SCALE64, sc);
-        for (int t = 1; t < nt; ++t) {
+        // P_t = D_0 A D_1 A ... D_t A, all of them: the prefix products of one chain.  In one launch (n <= 512):
+        // 40 slices at n = 98 in 148 us, 860 us as a GEMM per slice
+        const bool chain = chain_fits(n);
+        if (!chain) sc.push_back({A, D(0).re, D(0).im, mP(0).re, mP(0).im, n, SCALE_ROW});
+        if (!sc.empty()) b.add(K::SCALE64, sc);
+        if (chain) {
+            SuffixItem it{pk64_[species]->as<double>(), A, D(0).re, D(0).im, part, 2 * nn, 0, 1, nt, 1, 1};
+            it.keep = 1;
+            b.add(K::SUFFIX64, std::vector<SuffixItem>{it}, n, n);
+        }
+        for (int t = 1; t < nt && !chain; ++t) {
             std::vector<GemmItem<double>> gi{gitem<double>(mP(t - 1).re, mP(t - 1).im, A, nullptr, mP(t), D(t).re,
                                                            D(t).im, nullptr, nullptr, n)};
             b.add(K::GEMM64_CR_PRE, gi, n, n);
         }
         b.finish();
-        run(op, phi);
-        if (hop_ == DIA) {
-            // W_t = part_{t-1} D_t (the product without the final K)
+        sf_.products[species] = std::move(op);
+    }
+    if (!sf_.lu) {  // LU of every partial product (+1 on the last), in place; Mz keeps the products
+        std::vector<LuItem> lu;
+        for (int t = 0; t < nt; ++t) {
+            lu.push_back({mP(t).re, mP(t).im, sf_.piv->as<int>() + (long)t * n, nullptr,
+                          sf_.luw->as<double>() + t * lu_work_doubles(n), n, n});
+            lu.back().add = t == nt - 1;
+        }
+        std::unique_ptr<DevBuf> d(new DevBuf(lu.size() * sizeof(LuItem)));
+        ISLE_HIP(hipMemcpy(d->p, lu.data(), lu.size() * sizeof(LuItem), hipMemcpyHostToDevice));
+        if (hop_ == DIA && nt > 1) {  // W_t = part_{t-1} D_t (the product without the final K)
             std::vector<CScaleItem<double>> cs;
             for (int t = 1; t < nt; ++t)
                 cs.push_back({mP(t - 1).re, mP(t - 1).im, D(t).re, D(t).im, mM(t).re, mM(t).im, n, SCALE_COL});
-            if (!cs.empty()) {
-                DevBuf dcs(cs.size() * sizeof(CScaleItem<double>));
-                ISLE_HIP(hipMemcpy(dcs.p, cs.data(), cs.size() * sizeof(cs[0]), hipMemcpyHostToDevice));
-                hipLaunchKernelGGL(scale_complex_kernel<double>, dim3(ew_blocks(nn), cs.size()), dim3(EW_THREADS), 0,
-                                   s, dcs.as<CScaleItem<double>>());
-                ISLE_HIP(hipGetLastError());
-            }
-        } else {
-            ISLE_HIP(hipMemcpyAsync(Mz, part, (size_t)nt * 2 * nn * sizeof(double), hipMemcpyDeviceToDevice, s));
+            sf_.scale.reset(new DevBuf(cs.size() * sizeof(CScaleItem<double>)));
+            ISLE_HIP(hipMemcpy(sf_.scale->p, cs.data(), cs.size() * sizeof(cs[0]), hipMemcpyHostToDevice));
         }
-        // LU of every partial product (+1 on the last), in place; Mz keeps the products
-        std::vector<LuItem> lu;
-        for (int t = 0; t < nt; ++t)
-            lu.push_back({mP(t).re, mP(t).im, piv + (long)t * n, nullptr, luw_p + t * lu_work_doubles(n), n, n});
-        DevBuf dlu(lu.size() * sizeof(LuItem));
-        ISLE_HIP(hipMemcpy(dlu.p, lu.data(), lu.size() * sizeof(LuItem), hipMemcpyHostToDevice));
-        if (nt > 1) launch_lu(dlu.as<LuItem>(), nt - 1, n, 0, s);
-        launch_lu(dlu.as<LuItem>() + (nt - 1), 1, n, 1, s);
-        ISLE_HIP(hipStreamSynchronize(s));
-        sf_.nt = nt;
-        sf_.species = species;
+        sf_.lu = std::move(d);
     }
-    const long blk = 2L * n * nrhs;
-    // The slice products of the right-hand sides and the blocked triangular solves are launch
-    // steps with tuned tiles (once per shape: the plan caches the choice).  Tuning runs them
-    // on the workspace before it holds this call's data; the factorization is only read.
-    OpCache og;
-    og.nt = nt;
+    run(*sf_.products[species], phi);
+    if (hop_ == DIA) {
+        if (nt > 1) {
+            hipLaunchKernelGGL(scale_complex_kernel<double>, dim3(ew_blocks(nn), nt - 1), dim3(EW_THREADS), 0, s,
+                               sf_.scale->as<CScaleItem<double>>());
+            ISLE_HIP(hipGetLastError());
+        }
+    } else {
+        ISLE_HIP(hipMemcpyAsync(Mz, part, (size_t)nt * 2 * nn * sizeof(double), hipMemcpyDeviceToDevice, s));
+    }
+    launch_lu(sf_.lu->as<LuItem>(), nt, n, 0, s);
+    sf_.species = species;
+}
+
+// The launch descriptors of nrhs right-hand sides (workspace: Bt, Z, nt blocks of 2 n nrhs; Xl and a
+// scratch block).  The slice products of the right-hand sides and the blocked triangular solves are launch
+// steps with tuned tiles (once per shape: the plan caches the choice).  Tuning runs them on the workspace
+// before it holds this call's data; the factorization is only read.
+void Plan::solve_rhs(int nt, int nrhs, double* Bt) {
+    const int n = nx_;
+    const long nn = (long)n * n, blk = 2L * n * nrhs;
+    if (sf_.nrhs == nrhs && sf_.ws == Bt) return;
+    sf_.nrhs = -1;
+    double* part = sf_.part->as<double>();
+    double* Mz = sf_.mz->as<double>();  // matrices multiplying the rhs (EXP: a copy of the partial products)
+    int* piv = sf_.piv->as<int>();
+    double* luw_p = sf_.luw->as<double>();
+    double* Z = Bt + nt * blk;
+    double* Xl = Z + nt * blk;
+    double* Sc = Xl + blk;
+    auto mP = [&](int t) { return cmat(part, t, nn); };
+    auto mM = [&](int t) { return cmat(Mz, t, nn); };
+    auto fresh = [&] {
+        std::unique_ptr<OpCache> op(new OpCache);
+        op->nt = nt;
+        return op;
+    };
+    std::unique_ptr<OpCache> og = fresh();
     {
-        Builder bg(og);
+        Builder bg(*og);
         std::vector<GemmItem<double>> gi;
         for (int t = 0; t < nt; ++t) {
             GemmItem<double> g{};
@@ -2661,21 +2691,22 @@ void Plan::solveM(const double* phi, int nt, int species, const double* rhss, in
         }
         bg.add(K::GEMM64_CC, gi, n, nrhs);
         bg.finish();
-        tune(og);
+        tune(*og);
     }
     // many right-hand sides: the triangular solves as blocked GEMMs (rows gathered into
     // each LU's pivot order, then unit-lower and upper solves with the stored inverses of
     // the 32 x 32 diagonal blocks): o1 solves the last slice, o2 every slice
-    const bool blocked = n % LU_NB == 0 && nrhs >= 64;
-    OpCache o1, o2;
-    o1.nt = o2.nt = nt;
-    if (blocked) {
+    std::unique_ptr<OpCache> o1, o2;
+    std::unique_ptr<DevBuf> d1, d2;
+    if (solve_blocked(nrhs)) {
+        o1 = fresh();
+        o2 = fresh();
         auto lu_mat = [&](int t, double* rre, double* rim, double* xre, double* xim) {
             return TrsmMat{mP(t).re, mP(t).im, n, luw_p + t * lu_work_doubles(n), rre, rim, nrhs, xre, xim, nrhs};
         };
         auto rows = [&](double* p) { return std::make_pair(p, p + (long)n * nrhs); };
-        Builder b1(o1);
-        int* sig = b1.di((size_t)nt * n);  // o1 outlives o2, which reads it
+        Builder b1(*o1);
+        int* sig = b1.di((size_t)nt * n);  // o1 lives as long as o2, which reads it
         std::vector<SigmaItem> sv;
         for (int t = 0; t < nt; ++t) sv.push_back({piv + (long)t * n, sig + (long)t * n, n, n});
         b1.add(K::SIGMA, sv);
@@ -2686,7 +2717,7 @@ void Plan::solveM(const double* phi, int nt, int species, const double* rhss, in
         add_trsm(b1, 0, n, nrhs, {lu_mat(nt - 1, g0.first, g0.second, g1.first, g1.second)});
         add_trsm(b1, 1, n, nrhs, {lu_mat(nt - 1, g1.first, g1.second, xl.first, xl.second)});
         b1.finish();
-        Builder b2(o2);
+        Builder b2(*o2);
         std::vector<RowGatherItem> ra;
         std::vector<TrsmMat> tl, tu;
         for (int t = 0; t < nt; ++t) {
@@ -2699,63 +2730,85 @@ void Plan::solveM(const double* phi, int nt, int species, const double* rhss, in
         add_trsm(b2, 0, n, nrhs, tl);
         add_trsm(b2, 1, n, nrhs, tu);
         b2.finish();
-        tune(o1);
-        tune(o2);
+        tune(*o1);
+        tune(*o2);
+    } else {
+        auto sitem = [&](int t) {
+            SolveItem si{};
+            si.lu_re = mP(t).re;
+            si.lu_im = mP(t).im;
+            si.piv = piv + (long)t * n;
+            si.dinv = luw_p + t * lu_work_doubles(n);
+            si.b_re = Z + t * blk;
+            si.b_im = Z + t * blk + (long)n * nrhs;
+            si.bsr = nrhs;
+            si.bsc = 1;
+            si.n = n;
+            si.ld = n;
+            si.nrhs = nrhs;
+            return si;
+        };
+        auto upload = [&](const std::vector<SolveItem>& v) {
+            std::unique_ptr<DevBuf> d(new DevBuf(v.size() * sizeof(SolveItem)));
+            ISLE_HIP(hipMemcpy(d->p, v.data(), v.size() * sizeof(SolveItem), hipMemcpyHostToDevice));
+            return d;
+        };
+        SolveItem l = sitem(nt - 1);
+        l.x_re = Xl;
+        l.x_im = Xl + (long)n * nrhs;
+        l.xsr = nrhs;
+        l.xsc = 1;
+        d1 = upload({l});
+        std::vector<SolveItem> sv;  // the last slice solves the original z_{nt-1} again (Z is not modified there)
+        for (int t = 0; t < nt; ++t) {
+            sv.push_back(sitem(t));
+            sv.back().xoff = 2L * t * n;  // in the caller's array
+            sv.back().xsr = 2;
+            sv.back().xsc = 2L * nt * n;
+        }
+        d2 = upload(sv);
     }
+    sf_.rhs = std::move(og);
+    sf_.last = std::move(o1);
+    sf_.every = std::move(o2);
+    sf_.solve_last = std::move(d1);
+    sf_.solve_every = std::move(d2);
+    sf_.ws = Bt;
+    sf_.nrhs = nrhs;
+}
+
+// solveM (hubbardFermiMatrixExp.cpp:645-694, hubbardFermiMatrixDia.cpp:617-673).
+void Plan::solveM(const double* phi, int nt, int species, const double* rhss, int nrhs, double* out, bool reuse) {
+    const int n = nx_;
+    hipStream_t s = stream_;
+    if (!(reuse && sf_.nt == nt && sf_.species == species)) solve_factor(phi, nt, species);
+    const long blk = 2L * n * nrhs;
+    double* Bt = solve_workspace((2 * (size_t)nt + 2) * blk);
+    double* Z = Bt + nt * blk;
+    double* Xl = Z + nt * blk;
+    solve_rhs(nt, nrhs, Bt);
     const dim3 tgrid(cdiv(n, 32), cdiv(nrhs, 32), nt);
     hipLaunchKernelGGL(rhs_transpose_kernel, tgrid, dim3(256), 0, s, rhss, Bt, n, nt, nrhs);
     ISLE_HIP(hipGetLastError());
-    run(og, phi);
+    run(*sf_.rhs, phi);
     hipLaunchKernelGGL(prefix_sum_t_kernel, dim3(ew_blocks(blk)), dim3(EW_THREADS), 0, s, Z, blk, nt);
     ISLE_HIP(hipGetLastError());
-    if (blocked) {
-        run(o1, phi);  // x_{nt-1} = (1 + A^-1)^-1 z_{nt-1}
-        if (nt > 1) {
-            hipLaunchKernelGGL(sub_last_kernel, dim3(ew_blocks(blk * (nt - 1))), dim3(EW_THREADS), 0, s, Z, Xl, blk,
-                               nt - 1);
-            ISLE_HIP(hipGetLastError());
-        }
-        run(o2, phi);  // x_t = A_t^-1 (z_t - x_{nt-1}) (z_{nt-1} unchanged: solves x_{nt-1} again)
-        hipLaunchKernelGGL(rhs_untranspose_kernel, tgrid, dim3(256), 0, s, Bt, out, n, nt, nrhs);
-        ISLE_HIP(hipGetLastError());
-        ISLE_HIP(hipStreamSynchronize(s));
-        return;
-    }
-    ISLE_HIP(hipStreamSynchronize(s));
-    auto sitem = [&](int t, const double* bre, long bsr, long bsc, double* xre, double* xim, long xsr, long xsc) {
-        SolveItem si{};
-        si.lu_re = mP(t).re;
-        si.lu_im = mP(t).im;
-        si.piv = piv + (long)t * n;
-        si.dinv = luw_p + t * lu_work_doubles(n);
-        si.b_re = bre;
-        si.b_im = bre + (long)n * nrhs;
-        si.bsr = bsr;
-        si.bsc = bsc;
-        si.x_re = xre;
-        si.x_im = xim;
-        si.xsr = xsr;
-        si.xsc = xsc;
-        si.n = n;
-        si.ld = n;
-        si.nrhs = nrhs;
-        return si;
-    };
-    std::vector<SolveItem> s1{sitem(nt - 1, Z + (nt - 1) * blk, nrhs, 1, Xl, Xl + (long)n * nrhs, nrhs, 1)};
-    DevBuf ds1(sizeof(SolveItem));
-    ISLE_HIP(hipMemcpy(ds1.p, s1.data(), sizeof(SolveItem), hipMemcpyHostToDevice));
-    launch_lu_solve(ds1.as<SolveItem>(), 1, n, nrhs, s);
+    const bool blocked = solve_blocked(nrhs);
+    if (blocked)  // x_{nt-1} = (1 + A^-1)^-1 z_{nt-1}
+        run(*sf_.last, phi);
+    else
+        launch_lu_solve(sf_.solve_last->as<SolveItem>(), 1, n, nrhs, s);
     if (nt > 1) {
         hipLaunchKernelGGL(sub_last_kernel, dim3(ew_blocks(blk * (nt - 1))), dim3(EW_THREADS), 0, s, Z, Xl, blk, nt - 1);
         ISLE_HIP(hipGetLastError());
     }
-    std::vector<SolveItem> sv;
-    for (int t = 0; t < nt; ++t)
-        sv.push_back(sitem(t, Z + t * blk, nrhs, 1, out + 2L * t * n, out + 2L * t * n + 1, 2, 2L * nt * n));
-    // the last slice solves the original z_{nt-1} again (Z was not modified there)
-    DevBuf dsv(sv.size() * sizeof(SolveItem));
-    ISLE_HIP(hipMemcpy(dsv.p, sv.data(), sv.size() * sizeof(SolveItem), hipMemcpyHostToDevice));
-    launch_lu_solve(dsv.as<SolveItem>(), nt, n, nrhs, s);
+    if (blocked) {  // x_t = A_t^-1 (z_t - x_{nt-1}) (z_{nt-1} unchanged: solves x_{nt-1} again)
+        run(*sf_.every, phi);
+        hipLaunchKernelGGL(rhs_untranspose_kernel, tgrid, dim3(256), 0, s, Bt, out, n, nt, nrhs);
+        ISLE_HIP(hipGetLastError());
+    } else {
+        launch_lu_solve(sf_.solve_every->as<SolveItem>(), nt, n, nrhs, s, out);
+    }
     ISLE_HIP(hipStreamSynchronize(s));
 }
 

@@ -199,8 +199,16 @@ private:
     // solveM's factorization of the last field: phases, the matrices that multiply the
     // right-hand sides, the partial products' LUs (in place), pivots and LU work buffers
     struct SolveFactor {
-        int nt = -1, species = -1;
+        int nt = -1;       // time extent of the buffers
+        int species = -1;  // whose factorisation they hold (-1: none)
         std::unique_ptr<DevBuf> ph, mz, part, piv, luw;
+        // launch descriptors: they name the buffers above (and solve_ws_), never a caller's arrays
+        std::unique_ptr<OpCache> products[2];              // per species
+        std::unique_ptr<DevBuf> lu, scale;                 // LU items; DIA: mz_t = part_{t-1} D_t
+        std::unique_ptr<OpCache> rhs, last, every;         // for nrhs right-hand sides
+        std::unique_ptr<DevBuf> solve_last, solve_every;
+        int nrhs = -1;
+        const double* ws = nullptr;                        // solve_ws_ when they were made
     };
     SolveFactor sf_;
     // applyM's split-plane operands and GEMM descriptors, kept and grown like solve_ws_
@@ -209,6 +217,9 @@ private:
     int apply_items_n_ = 0;
     size_t solve_ws_doubles_ = 0;
     double* solve_workspace(size_t doubles);
+    void solve_factor(const double* phi, int nt, int species);
+    void solve_rhs(int nt, int nrhs, double* Bt);
+    bool solve_blocked(int nrhs) const { return nx_ % 32 == 0 && nrhs >= 64; }
 
     void build_exp(const std::vector<double>& x, DevBuf& out);
     OpCache& get_force_plain(int nt, int batch, int nspecies, int spin);
