@@ -128,6 +128,12 @@ int isle_applyM(isle_hfm* h, const double* phi, int nt, int species, const doubl
 int isle_qlu(isle_hfm* h, const double* phi, int nt, double* dinv, double* u, double* l, double* v, double* hh,
              double* logdet_host);
 
+/* log det Q (logdetQ, hubbardFermiMatrixExp.cpp:540-570) as the log dets of nt blocks, re and im
+ * (logdet_host: 2 nt doubles; their sum is log det Q up to the branch), nt >= 3: block cyclic
+ * reduction of Q, every other block at once, without the factors that isle_qlu returns.
+ * Synchronises the handle's stream once. */
+int isle_logdetq(isle_hfm* h, const double* phi, int nt, double* logdet_host);
+
 /* solveQ (hubbardFermiMatrixExp.cpp:494-537; bind_hubbardFermiMatrix.cpp:47-49) on the blocks of
  * Q's LU as isle_qlu returns them (device interleaved complex128: dinv [nt], u and l [nt-1], v and
  * h [nt-2] blocks of nx*nx): the forward substitution with l and h, then the backward one with

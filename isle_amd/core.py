@@ -462,9 +462,18 @@ def getQLU(hfm, phi):
 def logdetQ(hfm, phi=None):
     """log det Q(phi) = sum_i log det d_i, Im in [-pi, pi] (logdetQ,
     hubbardFermiMatrixExp.cpp:540-570, bind_hubbardFermiMatrix.cpp:44-46).
-    ``logdetQ(qlu)`` reuses a factorisation from getQLU."""
+    ``logdetQ(qlu)`` reuses a factorisation from getQLU; without one, for nt >= 3, the blocks
+    are eliminated natively by block cyclic reduction (isle_logdetq)."""
     if not isinstance(hfm, QLU) and phi is None:
         raise TypeError("logdetQ takes (hfm, phi) or (qlu)")
+    if not isinstance(hfm, QLU):
+        nx = hfm.nx()
+        phi = as_field(phi, nx)
+        nt = phi.shape[-1] // nx
+        if phi.dim() == 1 and nt >= 3:
+            ld = np.empty(2 * nt)
+            _lib.check(_lib.load().isle_logdetq(hfm.handle, _lib.ptr(phi.contiguous()), nt, _lib.dptr(ld)))
+            return to_first_log_branch(complex(ld[::2].sum(), ld[1::2].sum()))
     lu = hfm if isinstance(hfm, QLU) else getQLU(hfm, phi)
     if not lu.isConsistent():
         raise RuntimeError("Components of LU not initialized properly")

@@ -20,7 +20,7 @@
 namespace isle {
 
 // dst (rows x cols, row stride ldd, split re/im planes given separately) =
-//   mode 0: 0,  1: identity,  2: src,  3: -src  (src row stride lds)
+//   mode 0: 0,  1: identity,  2: src,  3: -src,  4: dst + src  (src row stride lds)
 struct BlockItem {
     double* d_re;
     double* d_im;
@@ -44,6 +44,9 @@ __global__ __launch_bounds__(256) void block_fill_kernel(const BlockItem* __rest
             if (it.mode == 3) {
                 vr = -vr;
                 vi = -vi;
+            } else if (it.mode == 4) {
+                vr += it.d_re[r * it.ldd + c];
+                vi += it.d_im[r * it.ldd + c];
             }
         }
         it.d_re[r * it.ldd + c] = vr;

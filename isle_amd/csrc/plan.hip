@@ -2127,36 +2127,11 @@ void Plan::force_parts_multi(int nops, const double* const* phis, const int* nts
     }
 }
 
-// Block LU of Q = M_p M_h^T (getQLU, hubbardFermiMatrixExp.cpp:419-479, the Dia file
-// repeats it), nt >= 3, as one cached operation: the off-diagonal blocks T+(t), T-(t) for all
-// t first (a real matrix, signed, times a phase vector on its rows or columns), then the
-// recursion, sequential in t:
-//   d_0 = P;  u_0 = T-(0), l_0 = T+(1) d_0^{-1}, v_0 = T+(0), h_0 = T-(nt-1) d_0^{-1}
-//   d_i = P - l_{i-1} u_{i-1};  l_i = T+(i+1) d_i^{-1}, h_i = -h_{i-1} u_{i-1} d_i^{-1},
-//         v_i = -l_{i-1} v_{i-1}, u_i = T-(i)                                  (1 <= i <= nt-3)
-//   d_{nt-2} = P - l_{nt-3} u_{nt-3};  u_{nt-2} = T-(nt-2) - l_{nt-3} v_{nt-3},
-//         l_{nt-2} = (T+(nt-1) - h_{nt-3} u_{nt-3}) d_{nt-2}^{-1}
-//   d_{nt-1} = P - l_{nt-2} u_{nt-2} - sum_i h_i v_i
-// Each d_i^{-1} comes from one LU with partial pivoting (its log det kept on the device)
-// and its triangular solves; products are complex GEMMs tuned per shape, with the four real
-// products of the textbook form (the Gauss form's larger error in the imaginary parts,
-// carried through the recursion and the final sum, moved log det Q by ~1e-8 relative at
-// Nx=288, Nt=128, against ~3e-10 for the four-product form).  The h_i are
-// stored side by side (one nx x (nt-2)nx matrix) and the v_i stacked, so the last sum is
-// one GEMM with k = (nt-2) nx.
-OpCache& Plan::get_qlu(int nt) {
-    if (nt < 3) throw std::invalid_argument("the native QLU needs nt >= 3");
-    auto key = std::make_tuple(7, nt, 0, 0, 0, 0);
-    auto found = cache_.find(key);
-    if (found != cache_.end()) return *found->second;
-    auto op = std::make_unique<OpCache>();
-    op->nt = nt;
-    op->batch = 1;
-    op->phi_stride = 2L * nx_ * nt;
-    Builder b(*op);
+// The blocks of Q for all t, as the first steps of an operation: P, and T+(t), T-(t) (row t's factors of
+// x_{t-1} and x_{t+1}, cyclic): a real matrix, signed, times a phase vector on its rows or columns.
+Plan::QBlocks Plan::add_q_blocks(Builder& b, int nt) {
     const int n = nx_;
     const long nn = (long)n * n;
-    const int nh = nt - 2;  // h and v blocks
     // real factors of the off-diagonal blocks, and P, on the host
     std::vector<double> rp(nn), rm(nn), pm(nn, 0.0);
     if (hop_ == EXP) {
@@ -2217,6 +2192,60 @@ OpCache& Plan::get_qlu(int nt) {
     };
     double* Tp = b.d64((size_t)nt * 2 * nn);
     double* Tm = b.d64((size_t)nt * 2 * nn);
+    auto tp = [&](int t) { return cmat(Tp, t, nn); };
+    auto tm = [&](int t) { return cmat(Tm, t, nn); };
+    std::vector<PhaseItem> phs = {{0, 0, 1.0, D(1, 0).re, D(1, 0).im, nullptr, nullptr, n, nt},
+                                  {0, 0, -1.0, D(-1, 0).re, D(-1, 0).im, nullptr, nullptr, n, nt}};
+    b.add(K::PHASE, phs);
+    {
+        std::vector<ScaleItem<double>> sc;
+        for (int t = 0; t < nt; ++t) {
+            // signs: EXP T+ is + at t = 0, T- + at t = nt-1, - elsewhere; DIA the opposite
+            const bool wrap_p = t == 0, wrap_m = t == nt - 1;
+            const bool neg_p = expo ? !wrap_p : wrap_p, neg_m = expo ? !wrap_m : wrap_m;
+            const double* ap = R + (neg_p ? nn : 0);
+            const double* am = R + 2 * nn + (neg_m ? nn : 0);
+            const CMat<double> dp = D(1, t), dm = D(-1, (t + 1) % nt);  // e^{i phi_{t-1}}, e^{-i phi_t}
+            sc.push_back({ap, dp.re, dp.im, tp(t).re, tp(t).im, n, expo ? SCALE_COL : SCALE_ROW});
+            sc.push_back({am, dm.re, dm.im, tm(t).re, tm(t).im, n, expo ? SCALE_ROW : SCALE_COL});
+        }
+        b.add(K::SCALE64, sc);
+    }
+    return {Pb, Tp, Tm};
+}
+
+// Block LU of Q = M_p M_h^T (getQLU, hubbardFermiMatrixExp.cpp:419-479, the Dia file
+// repeats it), nt >= 3, as one cached operation: the off-diagonal blocks T+(t), T-(t) for all
+// t first (a real matrix, signed, times a phase vector on its rows or columns), then the
+// recursion, sequential in t:
+//   d_0 = P;  u_0 = T-(0), l_0 = T+(1) d_0^{-1}, v_0 = T+(0), h_0 = T-(nt-1) d_0^{-1}
+//   d_i = P - l_{i-1} u_{i-1};  l_i = T+(i+1) d_i^{-1}, h_i = -h_{i-1} u_{i-1} d_i^{-1},
+//         v_i = -l_{i-1} v_{i-1}, u_i = T-(i)                                  (1 <= i <= nt-3)
+//   d_{nt-2} = P - l_{nt-3} u_{nt-3};  u_{nt-2} = T-(nt-2) - l_{nt-3} v_{nt-3},
+//         l_{nt-2} = (T+(nt-1) - h_{nt-3} u_{nt-3}) d_{nt-2}^{-1}
+//   d_{nt-1} = P - l_{nt-2} u_{nt-2} - sum_i h_i v_i
+// Each d_i^{-1} comes from one LU with partial pivoting (its log det kept on the device)
+// and its triangular solves; products are complex GEMMs tuned per shape, with the four real
+// products of the textbook form (the Gauss form's larger error in the imaginary parts,
+// carried through the recursion and the final sum, moved log det Q by ~1e-8 relative at
+// Nx=288, Nt=128, against ~3e-10 for the four-product form).  The h_i are
+// stored side by side (one nx x (nt-2)nx matrix) and the v_i stacked, so the last sum is
+// one GEMM with k = (nt-2) nx.
+OpCache& Plan::get_qlu(int nt) {
+    if (nt < 3) throw std::invalid_argument("the native QLU needs nt >= 3");
+    auto key = std::make_tuple(7, nt, 0, 0, 0, 0);
+    auto found = cache_.find(key);
+    if (found != cache_.end()) return *found->second;
+    auto op = std::make_unique<OpCache>();
+    op->nt = nt;
+    op->batch = 1;
+    op->phi_stride = 2L * nx_ * nt;
+    Builder b(*op);
+    const int n = nx_;
+    const long nn = (long)n * n;
+    const int nh = nt - 2;  // h and v blocks
+    const QBlocks q = add_q_blocks(b, nt);
+    double *Tp = q.tplus, *Tm = q.tminus, *Pb = q.p;
     // With n % 32 == 0: [d_i | 1] (n x 2n), whose LU over the first n columns leaves L^{-1} P
     // in the right block; otherwise d_i alone and both triangular solves
     const bool aug = n % LU_NB == 0;
@@ -2246,23 +2275,6 @@ OpCache& Plan::get_qlu(int nt) {
     const CMat<double> dw{Dw, Dw + dpl}, dr{Dw + n, Dw + dpl + n};  // d and (aug) the identity block
     const CMat<double> tw = cmat(tmp, 0, nn), pb = cmat(Pb, 0, nn);
 
-    std::vector<PhaseItem> phs = {{0, 0, 1.0, D(1, 0).re, D(1, 0).im, nullptr, nullptr, n, nt},
-                                  {0, 0, -1.0, D(-1, 0).re, D(-1, 0).im, nullptr, nullptr, n, nt}};
-    b.add(K::PHASE, phs);
-    {
-        std::vector<ScaleItem<double>> sc;
-        for (int t = 0; t < nt; ++t) {
-            // signs: EXP T+ is + at t = 0, T- + at t = nt-1, - elsewhere; DIA the opposite
-            const bool wrap_p = t == 0, wrap_m = t == nt - 1;
-            const bool neg_p = expo ? !wrap_p : wrap_p, neg_m = expo ? !wrap_m : wrap_m;
-            const double* ap = R + (neg_p ? nn : 0);
-            const double* am = R + 2 * nn + (neg_m ? nn : 0);
-            const CMat<double> dp = D(1, t), dm = D(-1, (t + 1) % nt);  // e^{i phi_{t-1}}, e^{-i phi_t}
-            sc.push_back({ap, dp.re, dp.im, tp(t).re, tp(t).im, n, expo ? SCALE_COL : SCALE_ROW});
-            sc.push_back({am, dm.re, dm.im, tm(t).re, tm(t).im, n, expo ? SCALE_ROW : SCALE_COL});
-        }
-        b.add(K::SCALE64, sc);
-    }
     auto cc = [&](CMat<double> a, long lda, CMat<double> bb, long ldb, CMat<double> c, long ldc, int k) {
         GemmItem<double> g{};
         g.a_re = a.re;
@@ -2390,6 +2402,162 @@ void Plan::qlu(const double* phi, int nt, double* dinv, double* u, double* l, do
     out(e[5], e[6], n, (long)(nt - 2) * n, nt - 2, h);
     ISLE_HIP(hipMemcpyAsync(logdet_host, op.logdet, 2 * sizeof(double) * nt, hipMemcpyDeviceToHost, s));
     ISLE_HIP(hipStreamSynchronize(s));
+}
+
+// log det Q alone (nt >= 3), by block cyclic reduction: Q is block-cyclic tridiagonal (row t: T+(t) x_{t-1}
+// + P_t x_t + T-(t) x_{t+1}), and every other block x_j is eliminated at once, X = P_j^{-1} [T+(j) | T-(j)]
+// = [Xp | Xm], leaving a system of the same form with half the blocks: with its neighbours a and c
+//   P_a -= T-(a) Xp,  T-'(a) = -T-(a) Xm,   P_c -= T+(c) Xm,  T+'(c) = -T+(c) Xp
+// (the same for a = c; with an odd number the last and the first stay neighbours), down to one block
+// P + T+ + T-.  Every P_j is factorised with partial pivoting within the block and products are of four
+// real ones, as in getQLU's recursion, whose nt factorisations are one after the other: it is their
+// sequence (LU panels of one matrix) that bounds log det Q, here log2(nt) + 1 of them over all blocks of a
+// level: 2.04 ms for n = 128, nt = 48 (15.4 ms by the recursion).  Its errors are those
+// of the recursion (ten fields, n 12 to 200, nt 9 to 45: 1e-15 to 2e-10, larger than its by 1.2 at most where
+// above 1e-13).
+OpCache& Plan::get_logdetq(int nt) {
+    if (nt < 3) throw std::invalid_argument("the native log det Q needs nt >= 3");
+    auto key = std::make_tuple(9, nt, 0, 0, 0, 0);
+    auto found = cache_.find(key);
+    if (found != cache_.end()) return *found->second;
+    auto op = std::make_unique<OpCache>();
+    op->nt = nt;
+    op->batch = 1;
+    op->phi_stride = 2L * nx_ * nt;
+    Builder b(*op);
+    const int n = nx_;
+    const long nn = (long)n * n;
+    const QBlocks qb = add_q_blocks(b, nt);
+    op->logdet = b.d64(2 * (size_t)nt);
+    // W = [P_j | T+(j) | T-(j)], its LU (n % 32 == 0: the LU carries the right-hand sides along, leaving the
+    // backward solve) and X, of the blocks that a level eliminates
+    const bool aug = n % LU_NB == 0;
+    const int nel = nt / 2;
+    const long ldw = 3L * n, ldx = 2L * n, wsz = 2 * n * ldw, xsz = 2 * n * ldx;
+    const size_t lwork = lu_work_doubles(n, (int)ldw);
+    double* W = b.d64((size_t)nel * wsz);
+    double* X = b.d64((size_t)nel * xsz);
+    double* work = b.d64((size_t)nel * lwork);
+    int* piv = b.di((size_t)nel * n);
+    auto w = [&](int k, int col) {
+        double* r = W + k * wsz + (long)col * n;
+        return CMat<double>{r, r + n * ldw};
+    };
+    auto x = [&](int k, int col) {
+        double* r = X + k * xsz + (long)col * n;
+        return CMat<double>{r, r + n * ldx};
+    };
+    struct Row {
+        CMat<double> p, tp, tm;
+    };
+    std::vector<Row> rows;
+    for (int t = 0; t < nt; ++t) rows.push_back({cmat(qb.p, 0, nn), cmat(qb.tplus, t, nn), cmat(qb.tminus, t, nn)});
+    auto fill = [&](std::vector<BlockItem>& v, const CMat<double>& d, long ldd, const CMat<double>& src, int mode) {
+        v.push_back({d.re, d.im, src.re, src.im, ldd, n, n, n, mode});
+    };
+    auto sub = [&](std::vector<GemmItem<double>>& v, const CMat<double>& a, const CMat<double>& c, const CMat<double>& xk) {
+        GemmItem<double> g{};  // c -= a xk
+        g.a_re = a.re;
+        g.a_im = a.im;
+        g.b_re = xk.re;
+        g.b_im = xk.im;
+        g.c_re = c.re;
+        g.c_im = c.im;
+        g.m = g.n = g.k = n;
+        g.lda = g.ldc = n;
+        g.ldb = (int)ldx;
+        v.push_back(g);
+    };
+    auto factorise = [&](int count, int slot, int nrhs) {  // W of blocks 0 .. count-1, log dets from `slot` on
+        const int ncols = aug ? n + nrhs : n;
+        std::vector<LuItem> lu;
+        std::vector<SolveItem> sv;
+        for (int k = 0; k < count; ++k) {
+            LuItem li{w(k, 0).re, w(k, 0).im, piv + (long)k * n, op->logdet + 2L * (slot + k), work + k * lwork, n, (int)ldw};
+            li.m = n;
+            li.ncols = ncols;
+            li.kf = n;
+            lu.push_back(li);
+            SolveItem si{};
+            si.lu_re = li.re;
+            si.lu_im = li.im;
+            si.piv = li.piv;
+            si.dinv = li.work;
+            si.b_re = w(k, 1).re;
+            si.b_im = w(k, 1).im;
+            si.bsr = ldw;
+            si.bsc = 1;
+            si.mode = aug ? (int)SOLVE_U : 7;
+            si.x_re = x(k, 0).re;
+            si.x_im = x(k, 0).im;
+            si.xsr = ldx;
+            si.xsc = 1;
+            si.n = n;
+            si.ld = (int)ldw;
+            si.nrhs = nrhs;
+            sv.push_back(si);
+        }
+        b.add(K::LU_SHAPE, lu, n, ncols, n, 0);
+        if (nrhs > 0) b.add(K::SOLVE, sv, n, nrhs);
+    };
+    int slot = 0;
+    const CMat<double> none{nullptr, nullptr};
+    while (rows.size() > 1) {
+        const int N = (int)rows.size(), ne = N / 2;  // eliminated: rows 1, 3, ..
+        std::vector<BlockItem> v;
+        std::vector<GemmItem<double>> up, down;  // both subtract from a kept row's P: one after the other
+        std::vector<Row> kept;
+        for (int t = 0; t < N; t += 2) {
+            Row r = rows[t];
+            const bool right = t + 1 < N, left = t > 0 || N % 2 == 0;  // an eliminated neighbour there
+            const int kr = t / 2, kl = t > 0 ? t / 2 - 1 : ne - 1;
+            r.p = cmat(b.d64(2 * nn), 0, nn);
+            fill(v, r.p, n, rows[t].p, 2);
+            if (right) {
+                r.tm = cmat(b.d64(2 * nn), 0, nn);
+                fill(v, r.tm, n, none, 0);
+                sub(up, rows[t].tm, r.p, x(kr, 0));
+                sub(up, rows[t].tm, r.tm, x(kr, 1));
+            }
+            if (left) {
+                r.tp = cmat(b.d64(2 * nn), 0, nn);
+                fill(v, r.tp, n, none, 0);
+                sub(down, rows[t].tp, r.p, x(kl, 1));
+                sub(down, rows[t].tp, r.tp, x(kl, 0));
+            }
+            kept.push_back(r);
+        }
+        for (int k = 0; k < ne; ++k) {
+            const Row& r = rows[2 * k + 1];
+            fill(v, w(k, 0), ldw, r.p, 2);
+            fill(v, w(k, 1), ldw, r.tp, 2);
+            fill(v, w(k, 2), ldw, r.tm, 2);
+        }
+        b.add(K::BLOCK, v, 0, 0, 0, (int)nn);
+        factorise(ne, slot, 2 * n);
+        slot += ne;
+        b.add(K::GEMM64_CC4_SUB, up, n, n);
+        b.add(K::GEMM64_CC4_SUB, down, n, n);
+        rows = std::move(kept);
+    }
+    for (const CMat<double>& m : {rows[0].p, rows[0].tp, rows[0].tm}) {
+        std::vector<BlockItem> v;
+        fill(v, w(0, 0), ldw, m, m.re == rows[0].p.re ? 2 : 4);
+        b.add(K::BLOCK, v, 0, 0, 0, (int)nn);
+    }
+    factorise(1, slot, 0);
+    b.finish();
+    tune(*op);
+    auto& ref = *op;
+    cache_[key] = std::move(op);
+    return ref;
+}
+
+void Plan::logdet_q(const double* phi, int nt, double* logdet_host) {
+    OpCache& op = get_logdetq(nt);
+    run(op, phi);
+    ISLE_HIP(hipMemcpyAsync(logdet_host, op.logdet, 2 * sizeof(double) * nt, hipMemcpyDeviceToHost, stream_));
+    ISLE_HIP(hipStreamSynchronize(stream_));
 }
 
 // solveQ (hubbardFermiMatrixExp.cpp:494-537) on the blocks of Q's LU, as one cached operation
@@ -3031,6 +3199,13 @@ int isle_qlu(isle_hfm* h, const double* phi, int nt, double* dinv, double* u, do
     return guarded([&] {
         if (nt < 3) throw std::invalid_argument("isle_qlu needs nt >= 3");
         P(h)->qlu(phi, nt, dinv, u, l, v, hh, logdet_host);
+    });
+}
+
+int isle_logdetq(isle_hfm* h, const double* phi, int nt, double* logdet_host) {
+    return guarded([&] {
+        if (nt < 3) throw std::invalid_argument("isle_logdetq needs nt >= 3");
+        P(h)->logdet_q(phi, nt, logdet_host);
     });
 }
 

@@ -155,6 +155,8 @@ public:
     // and log det d_i to logdet_host (nt x 2); one synchronisation at the end.
     void qlu(const double* phi, int nt, double* dinv, double* u, double* l, double* v, double* h,
              double* logdet_host);
+    // log det Q as nt log dets of blocks (their sum; nt x 2), without Q's LU; nt >= 3.
+    void logdet_q(const double* phi, int nt, double* logdet_host);
     // x with Q x = rhs from the blocks of Q's LU (interleaved complex128 device stacks as
     // getQLU returns them); rhs, x: nrhs x (nt * nx) rows.  nt >= 1.
     void solve_q(int nt, int nrhs, const double* dinv, const double* u, const double* l, const double* v,
@@ -239,7 +241,12 @@ private:
     OpCache& get_logdet_grouped(int nt, int batch, int group, int nspecies, int spin);
     OpCache& get_force_stable(int nt, int batch, int group, int nspecies, int spin, bool right32 = false);
     OpCache& get_logdet_stable(int nt, int batch, int group, int nspecies, int spin);
+    struct QBlocks {
+        double *p, *tplus, *tminus;  // P; T+(t), T-(t) (re plane, im plane, nt of each)
+    };
+    QBlocks add_q_blocks(Builder& b, int nt);
     OpCache& get_qlu(int nt);
+    OpCache& get_logdetq(int nt);
     OpCache& get_solveq(int nt, int nrhs);
     void run(OpCache& op, const double* phi, double* out = nullptr);
     bool launch_step(OpCache& op, const Step& st, const double* phi, double* out = nullptr);
