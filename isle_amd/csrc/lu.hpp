@@ -12,12 +12,13 @@
 //   lu_step_kernel   one workgroup per matrix (the chain that the whole factorisation waits for) first
 //                    takes the elimination of the panel before on the next panel's own columns, then
 //                    factorises that panel (one matrix row per thread, held in registers) with its
-//                    L11^{-1} and U11^{-1} and, on the item's last panel, the log-determinant; beside it
+//                    L11^{-1} and, on the item's last panel, U11^{-1} and the log-determinant; beside it
 //                    one workgroup per strip of LU_NB further columns takes the elimination of the panel
-//                    before there (interchanges, U12 = L11^{-1} A12, A22 -= L21 U12 on FP64 MFMA), and
-//                    more take its interchanges on the columns that are finished or not eliminated.
+//                    before there (interchanges, U12 = L11^{-1} A12, A22 -= L21 U12 on FP64 MFMA), one
+//                    its U11^{-1}, which only solves need, and more take its interchanges on the columns
+//                    that are finished or not eliminated.
 // Against a launch each for the panel, the interchanges and tiles of the elimination: order 288,
-// 704 -> 555 us for 32 matrices, 560 -> 526 us for one; order 128, 250 -> 213 us for 32.  Panels of more than LU_MAX_N candidate rows are factorised in global
+// 704 -> 529 us for 32 matrices, 560 -> 500 us for one; order 128, 250 -> 203 us for 32.  Panels of more than LU_MAX_N candidate rows are factorised in global
 // memory (lu_panel_tall_kernel) and keep those launches (lu_rswap_kernel, lu_update_kernel): a strip of
 // so many rows is too much work for one workgroup, and few strips would leave CUs idle.
 //
@@ -112,30 +113,36 @@ __device__ __forceinline__ unsigned long long pivot_key(double v, int pos) {
            static_cast<unsigned long long>(511 - pos);
 }
 
-// One DPP step on a 64-bit value: both halves move with the same lane pattern, so the
-// result is always some lane's whole value (or 0 where the pattern has no source lane).
+// Maximum of a 32-bit value over the 64 lanes of a wave, in registers: prefix maxima within each row of 16
+// lanes (row_shr 1, 2, 4, 8), then row 0's maximum into row 1 and row 2's into row 3 (row_bcast:15), then
+// lane 31's into rows 2 and 3 (row_bcast:31); lane 63 ends with the wave's maximum, which every lane reads.
 template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ unsigned long long dpp_u64(unsigned long long v) {
-    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROW_MASK, 0xf, true);
-    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, ROW_MASK, 0xf, true);
-    return ((unsigned long long)hi << 32) | lo;
+__device__ __forceinline__ unsigned dpp_max_u32(unsigned v) {
+    return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xf, true));
+}
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
+    v = dpp_max_u32<0x111, 0xf>(v);
+    v = dpp_max_u32<0x112, 0xf>(v);
+    v = dpp_max_u32<0x114, 0xf>(v);
+    v = dpp_max_u32<0x118, 0xf>(v);
+    v = dpp_max_u32<0x142, 0xa>(v);
+    v = dpp_max_u32<0x143, 0xc>(v);
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// Maximum of a non-negative 64-bit key over the 64 lanes of a wave, in registers: prefix
-// maxima within each row of 16 lanes (row_shr 1, 2, 4, 8), then row 0's maximum into row 1
-// and row 2's into row 3 (row_bcast:15), then lane 31's into rows 2 and 3 (row_bcast:31);
-// lane 63 ends with the wave's maximum, which every lane reads.
+// Maximum of a non-negative 64-bit key over the wave: of the high halves, then of the low halves where
+// the high half is that (mostly one lane: its value as it is).  All lanes active.  32 LUs of order 288: 552 us
+// with a 64-bit maximum by DPP (237 cycles in each of a panel's 32 column steps), 541 us so.
 __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long k) {
-    unsigned long long o;
-    o = dpp_u64<0x111, 0xf>(k); k = o > k ? o : k;
-    o = dpp_u64<0x112, 0xf>(k); k = o > k ? o : k;
-    o = dpp_u64<0x114, 0xf>(k); k = o > k ? o : k;
-    o = dpp_u64<0x118, 0xf>(k); k = o > k ? o : k;
-    o = dpp_u64<0x142, 0xa>(k); k = o > k ? o : k;
-    o = dpp_u64<0x143, 0xc>(k); k = o > k ? o : k;
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)k, 63);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(k >> 32), 63);
-    return ((unsigned long long)hi << 32) | lo;
+    const unsigned hi = (unsigned)(k >> 32), lo = (unsigned)k;
+    const unsigned mh = wave_max_u32(hi);
+    const unsigned long long at = __ballot(hi == mh);
+    unsigned ml;
+    if (__popcll(at) == 1)
+        ml = (unsigned)__builtin_amdgcn_readlane((int)lo, (int)__ffsll((long long)at) - 1);
+    else
+        ml = wave_max_u32(hi == mh ? lo : 0u);
+    return ((unsigned long long)mh << 32) | ml;
 }
 
 // a_j += m b_j for complex a_j, b_j, j = 0 .. 3, with b_j taken from lane J + j of the 16 lanes that share
@@ -179,12 +186,12 @@ __device__ __forceinline__ void st_global2(double* p, double2 v) {
 }
 __device__ __forceinline__ void lu_wave_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// L11^{-1} and U11^{-1} of a factorised panel by recursive doubling (lt: L11 unit lower,
+// L11^{-1} (LOWER) and U11^{-1} (UPPER) of a factorised panel by recursive doubling (lt: L11 unit lower,
 // ut: U11 with its diagonal already inverted, both [NB][NB + 1] in LDS, tl / tu temporaries),
 // then written to the panel's slots of the work buffer.  Ends with a barrier-free copy; the
 // caller's threads must all take part (block-wide loops and barriers inside).
 //   [A 0; C D]^{-1} = [A^-1 0; -D^-1 C A^-1  D^-1],  [A B; 0 D]^{-1} = [A^-1 -A^-1 B D^-1; 0 D^-1]
-template <int NB>
+template <int NB, bool LOWER, bool UPPER>
 __device__ void lu_invert_panel_blocks(const LuItem& it, int panel, double (*lt_re)[NB + 1], double (*lt_im)[NB + 1],
                                        double (*ut_re)[NB + 1], double (*ut_im)[NB + 1], double (*tl_re)[NB + 1],
                                        double (*tl_im)[NB + 1], double (*tu_re)[NB + 1], double (*tu_im)[NB + 1]) {
@@ -200,23 +207,27 @@ __device__ void lu_invert_panel_blocks(const LuItem& it, int panel, double (*lt_
             double tr = 0, ti = 0, sr = 0, si = 0;
 #pragma unroll 8
             for (int q = 0; q < b; ++q) {
-                {  // C A^-1: terms q >= j
+                if (LOWER) {  // C A^-1: terms q >= j
                     const double cr = lt_re[o + b + i][o + q], ci = lt_im[o + b + i][o + q];
                     const double xr = lt_re[o + q][o + j], xi = lt_im[o + q][o + j];
                     tr += q >= j ? cr * xr - ci * xi : 0.0;
                     ti += q >= j ? cr * xi + ci * xr : 0.0;
                 }
-                {  // B D^-1: terms q <= j
+                if (UPPER) {  // B D^-1: terms q <= j
                     const double br = ut_re[o + i][o + b + q], bi = ut_im[o + i][o + b + q];
                     const double xr = ut_re[o + b + q][o + b + j], xi = ut_im[o + b + q][o + b + j];
                     sr += q <= j ? br * xr - bi * xi : 0.0;
                     si += q <= j ? br * xi + bi * xr : 0.0;
                 }
             }
-            tl_re[o + b + i][o + j] = tr;
-            tl_im[o + b + i][o + j] = ti;
-            tu_re[o + i][o + b + j] = sr;
-            tu_im[o + i][o + b + j] = si;
+            if (LOWER) {
+                tl_re[o + b + i][o + j] = tr;
+                tl_im[o + b + i][o + j] = ti;
+            }
+            if (UPPER) {
+                tu_re[o + i][o + b + j] = sr;
+                tu_im[o + i][o + b + j] = si;
+            }
         }
         __syncthreads();
         for (int e = tid; e < work; e += nth) {
@@ -224,23 +235,27 @@ __device__ void lu_invert_panel_blocks(const LuItem& it, int panel, double (*lt_
             double xr_ = 0, xi_ = 0, yr = 0, yi = 0;
 #pragma unroll 8
             for (int q = 0; q < b; ++q) {
-                {  // D^-1 (C A^-1): terms q <= i
+                if (LOWER) {  // D^-1 (C A^-1): terms q <= i
                     const double dr = lt_re[o + b + i][o + b + q], di = lt_im[o + b + i][o + b + q];
                     const double tr = tl_re[o + b + q][o + j], ti = tl_im[o + b + q][o + j];
                     xr_ += q <= i ? dr * tr - di * ti : 0.0;
                     xi_ += q <= i ? dr * ti + di * tr : 0.0;
                 }
-                {  // A^-1 (B D^-1): terms q >= i
+                if (UPPER) {  // A^-1 (B D^-1): terms q >= i
                     const double ar_ = ut_re[o + i][o + q], ai_ = ut_im[o + i][o + q];
                     const double tr = tu_re[o + q][o + b + j], ti = tu_im[o + q][o + b + j];
                     yr += q >= i ? ar_ * tr - ai_ * ti : 0.0;
                     yi += q >= i ? ar_ * ti + ai_ * tr : 0.0;
                 }
             }
-            lt_re[o + b + i][o + j] = -xr_;
-            lt_im[o + b + i][o + j] = -xi_;
-            ut_re[o + i][o + b + j] = -yr;
-            ut_im[o + i][o + b + j] = -yi;
+            if (LOWER) {
+                lt_re[o + b + i][o + j] = -xr_;
+                lt_im[o + b + i][o + j] = -xi_;
+            }
+            if (UPPER) {
+                ut_re[o + i][o + b + j] = -yr;
+                ut_im[o + i][o + b + j] = -yi;
+            }
         }
         __syncthreads();
     }
@@ -249,10 +264,14 @@ __device__ void lu_invert_panel_blocks(const LuItem& it, int panel, double (*lt_
     double* ui_re = lu_uinv(it, panel);
     double* ui_im = ui_re + NB * NB;
     for (int e = tid; e < NB * NB; e += nth) {
-        li_re[e] = lt_re[e / NB][e % NB];
-        li_im[e] = lt_im[e / NB][e % NB];
-        ui_re[e] = ut_re[e / NB][e % NB];
-        ui_im[e] = ut_im[e / NB][e % NB];
+        if (LOWER) {
+            li_re[e] = lt_re[e / NB][e % NB];
+            li_im[e] = lt_im[e / NB][e % NB];
+        }
+        if (UPPER) {
+            ui_re[e] = ut_re[e / NB][e % NB];
+            ui_im[e] = ut_im[e / NB][e % NB];
+        }
     }
 }
 
@@ -446,6 +465,29 @@ __device__ inline void lu_strip_update(const LuItem& it, int kp, int c0, double*
     __syncthreads();
 }
 
+// U11^{-1} of the panel at kp, by one workgroup with 4 NB (NB + 1) doubles of LDS.
+template <int NB>
+__device__ inline void lu_invert_upper(const LuItem& it, int kp, double* lds) {
+    double(*ut_re)[NB + 1] = reinterpret_cast<double(*)[NB + 1]>(lds);
+    double(*ut_im)[NB + 1] = ut_re + NB;
+    double(*tu_re)[NB + 1] = ut_im + NB;
+    double(*tu_im)[NB + 1] = tu_re + NB;
+    for (int e = threadIdx.x; e < NB * NB; e += blockDim.x) {
+        const int r = e / NB, c = e % NB;
+        const long o = (long)(kp + r) * it.ld + kp + c;
+        double vr = it.re[o], vi = it.im[o];
+        if (r == c) {
+            const double den = vr * vr + vi * vi;
+            vr = vr / den;
+            vi = -vi / den;
+        }
+        ut_re[r][c] = c >= r ? vr : 0.0;
+        ut_im[r][c] = c >= r ? vi : 0.0;
+    }
+    __syncthreads();
+    lu_invert_panel_blocks<NB, false, true>(it, kp / NB, nullptr, nullptr, ut_re, ut_im, nullptr, nullptr, tu_re, tu_im);
+}
+
 // Rows of a wave between row-per-lane registers and coalesced memory accesses: a wave's 64 rows of
 // LU_TC columns of one plane in LDS, padded to 16 bytes off a power of two.
 constexpr int LU_TC = 16, LU_TROW = LU_TC + 2;
@@ -453,7 +495,7 @@ constexpr int LU_TC = 16, LU_TROW = LU_TC + 2;
 // One step of the factorisation: the panel at k0 (-1: none) of every item, and the elimination of the panel
 // at kp (-1: none) on the columns from cs on.  grid.x: nitems panel workgroups if k0 >= 0, then for each
 // unit one workgroup per item: `strips` of LU_NB columns, `defer` of LU_SWAP_COLS columns that take the
-// interchanges only, then the columns left of kp.  Items vary fastest, so the units of an item run on
+// interchanges only, kp's U11^{-1}, then the columns left of kp.  Items vary fastest, so the units of an item run on
 // its panel's XCD (L21 and the record come from its L2) when their number is a multiple of 8.  The
 // workgroups of one launch write disjoint columns and read, besides their own, only those of panel kp.
 template <int NB>
@@ -490,9 +532,11 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
         } else if (unit < strips + defer) {
             const int c = cd + LU_SWAP_COLS * (unit - strips);
             if (c < lu_ncols(it)) lu_swap_columns(it, kp, c, lu_ncols(it));
-        } else {
-            const int c = LU_SWAP_COLS * (unit - strips - defer);
+        } else if (unit > strips + defer) {
+            const int c = LU_SWAP_COLS * (unit - strips - defer - 1);
             if (c < kp) lu_swap_columns(it, kp, c, kp);
+        } else if (kp + NB < kf) {
+            lu_invert_upper<NB>(it, kp, big);
         }
         return;
     }
@@ -797,7 +841,11 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
     if (tid == 0) perm[0] = cnt;
     __syncthreads();
 
-    lu_invert_panel_blocks<NB>(it, panel, lt_re, lt_im, ut_re, ut_im, tl_re, tl_im, tu_re, tu_im);
+    if (k0 + NB < kf) {
+        lu_invert_panel_blocks<NB, true, false>(it, panel, lt_re, lt_im, ut_re, ut_im, tl_re, tl_im, tu_re, tu_im);
+        return;
+    }
+    lu_invert_panel_blocks<NB, true, true>(it, panel, lt_re, lt_im, ut_re, ut_im, tl_re, tl_im, tu_re, tu_im);
     lu_panel_logdet(it, k0, NB, kf, rsum);
 }
 
@@ -957,7 +1005,7 @@ __global__ __launch_bounds__(LU_TALL_THREADS) void lu_panel_tall_kernel(const Lu
         }
     }
     __syncthreads();
-    lu_invert_panel_blocks<NB>(it, panel, lt_re, lt_im, ut_re, ut_im, tl_re, tl_im, tu_re, tu_im);
+    lu_invert_panel_blocks<NB, true, true>(it, panel, lt_re, lt_im, ut_re, ut_im, tl_re, tl_im, tu_re, tu_im);
     lu_panel_logdet(it, k0, NB, kf, rsum);
 }
 
@@ -1208,7 +1256,8 @@ inline void launch_lu_shape(const LuItem* d_items, int nitems, int m, int ncols,
         const int strips = kp >= 0 ? std::max(0, nu - cs + LU_NB - 1) / LU_NB : 0;
         const int cd = std::max(cs, nu), defer = kp >= 0 ? std::max(0, ncols - cd + LU_SWAP_COLS - 1) / LU_SWAP_COLS : 0;
         const int left = kp >= 0 ? (kp + LU_SWAP_COLS - 1) / LU_SWAP_COLS : 0;
-        const int units = (k0 >= 0 ? 1 : 0) + strips + defer + left;
+        const int upper = kp >= 0 && kp + LU_NB < kf ? 1 : 0;  // U11^{-1} of kp, if not its last panel's
+        const int units = (k0 >= 0 ? 1 : 0) + strips + defer + (left > 0 ? 1 : upper) + left;
         if (units == 0) return;
         const int rows = lu_rows(kp >= 0 ? kp : k0, m, nt);
         // at least 4 waves: the strips and the inversion of L11 and U11 take that many
