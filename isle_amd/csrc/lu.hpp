@@ -18,9 +18,11 @@
 //                    its U11^{-1}, which only solves need, and more take its interchanges on the columns
 //                    that are finished or not eliminated.
 // Against a launch each for the panel, the interchanges and tiles of the elimination: order 288,
-// 704 -> 529 us for 32 matrices, 560 -> 500 us for one; order 128, 250 -> 203 us for 32.  Panels of more than LU_MAX_N candidate rows are factorised in global
-// memory (lu_panel_tall_kernel) and keep those launches (lu_rswap_kernel, lu_update_kernel): a strip of
-// so many rows is too much work for one workgroup, and few strips would leave CUs idle.
+// 704 -> 529 us for 32 matrices, 560 -> 500 us for one; order 128, 250 -> 203 us for 32.  Panels of more
+// than LU_MAX_N candidate rows keep those launches (lu_rswap_kernel, lu_update_kernel): a strip of so many
+// rows is too much work for one workgroup, and few strips would leave CUs idle.  Up to LU_MID_N rows their
+// panel is the same kernel's, with 12 waves and a third of the registers in scratch (90 us a panel; order 768,
+// two matrices: 10.1 -> 1.9 ms), beyond that in global memory (lu_panel_tall_kernel, 930 us).
 //
 // Besides square matrices the same kernels factorise the first kf columns of an m x ncols
 // matrix whose rows [k0+NB, nt) are, in the columns not yet factorised, known to be rows of
@@ -36,7 +38,8 @@
 namespace isle {
 
 constexpr int LU_NB = 32;          // panel width
-constexpr int LU_MAX_N = 512;      // one panel row per thread
+constexpr int LU_MAX_N = 512;      // one panel row per thread, elimination of the panel before beside it
+constexpr int LU_MID_N = 768;      // one panel row per thread, the panel alone
 constexpr int LU_UPD_THREADS = 256;
 constexpr int LU_TILE = 32;        // trailing-update tile
 constexpr int LU_SWAP_COLS = 64;   // columns per left-interchange workgroup
@@ -105,12 +108,14 @@ __device__ inline double block_sum(double v, double* s) {
 }
 
 // Pivot key: the bits of |re|+|im| (a non-negative double, so its bit pattern orders like
-// its value) with the low 9 mantissa bits replaced by 511 - position.  The maximal key is
-// the largest candidate, ties (and values equal to 2^-43 relative) going to the first
-// position, as izamax.  Positions must be < 512.
+// its value) with the low BITS mantissa bits replaced by 2^BITS - 1 - position.  The maximal key is
+// the largest candidate, ties (and values equal to 2^(BITS - 52) relative) going to the first
+// position, as izamax.  Positions must be < 2^BITS.
+template <int BITS>
 __device__ __forceinline__ unsigned long long pivot_key(double v, int pos) {
-    return (static_cast<unsigned long long>(__double_as_longlong(v)) & ~0x1FFull) |
-           static_cast<unsigned long long>(511 - pos);
+    constexpr int M = (1 << BITS) - 1;
+    return (static_cast<unsigned long long>(__double_as_longlong(v)) & ~static_cast<unsigned long long>(M)) |
+           static_cast<unsigned long long>(M - pos);
 }
 
 // Maximum of a 32-bit value over the 64 lanes of a wave, in registers: prefix maxima within each row of 16
@@ -498,10 +503,12 @@ constexpr int LU_TC = 16, LU_TROW = LU_TC + 2;
 // interchanges only, kp's U11^{-1}, then the columns left of kp.  Items vary fastest, so the units of an item run on
 // its panel's XCD (L21 and the record come from its L2) when their number is a multiple of 8.  The
 // workgroups of one launch write disjoint columns and read, besides their own, only those of panel kp.
-template <int NB>
-__global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restrict__ items, int nitems, int k0,
+template <int NB, int ROWS>
+__global__ __launch_bounds__(ROWS) void lu_step_kernel(const LuItem* __restrict__ items, int nitems, int k0,
                                                            int add_identity, int kp, int cs, int strips, int defer) {
-    constexpr int CG = 8, MAXW = LU_MAX_N / 64;  // columns per group, waves
+    constexpr int CG = 8, MAXW = ROWS / 64;  // columns per group, waves
+    constexpr int BITS = ROWS <= 512 ? 9 : 10;   // of a position
+    constexpr bool FUSED = ROWS <= LU_MAX_N;     // strips and the others units beside the panels
     static_assert(NB % LU_TC == 0 && NB % CG == 0, "columns go in groups");
     constexpr int TRI = NB * (NB + 1);           // one NB x (NB + 1) plane
     // one after the other: the waves' transposes of the loads, of the stores; then L11 / U11 and the
@@ -516,7 +523,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
     __shared__ double rsum[MAXW];
     // after the column loop: matrix row of each thread's row (80 KB in all: two workgroups on a CU)
     int* drow = reinterpret_cast<int*>(&gu12[0][0]);
-    static_assert(sizeof(gu12) >= LU_MAX_N * sizeof(int), "row numbers in the place of U12");
+    static_assert(sizeof(gu12) >= ROWS * sizeof(int), "row numbers in the place of U12");
 
     // `big` before the panel's own rows: U12 of the panel at kp and its row positions
     unsigned short* from = reinterpret_cast<unsigned short*>(big + LU_STRIP_LDS);
@@ -524,7 +531,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
     const int item = blockIdx.x % nitems, unit = blockIdx.x / nitems - (k0 >= 0 ? 1 : 0);
     const LuItem it = items[item];
     const int n = it.n, m = lu_m(it), kf = lu_kf(it), ntop = it.nt;
-    if (unit >= 0) {  // the panel at kp on the other columns (uniform over the workgroup)
+    if (FUSED && unit >= 0) {  // the panel at kp on the other columns (uniform over the workgroup)
         if (kp >= kf) return;
         const int ce = lu_nupd(it), cd = max(cs, ce);  // columns cs .. ce take the elimination, cd .. the interchanges
         if (unit < strips) {
@@ -541,7 +548,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
         return;
     }
     if (k0 >= kf) return;
-    if (kp >= 0) lu_strip_update(it, kp, k0, big, from);
+    if (FUSED && kp >= 0) lu_strip_update(it, kp, k0, big, from);
     const int ld = it.ld, tid = threadIdx.x, nth = blockDim.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rows = lu_rows(k0, m, ntop), kb = min(NB, kf - k0);
@@ -639,13 +646,13 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
             if (kk < kb) {
                 {  // max over the wave first (lanes to one LDS address serialise), then one atomic per wave
                     const unsigned long long key =
-                        wave_max_u64((own && pos >= kk) ? pivot_key(cabs1(ar[Q], ai[Q]), pos) : 0ull);
+                        wave_max_u64((own && pos >= kk) ? pivot_key<BITS>(cabs1(ar[Q], ai[Q]), pos) : 0ull);
                     if ((tid & 63) == 0 && key != 0ull) atomicMax(&pkey[kk], key);
                 }
                 __syncthreads();
                 // pivot position; an exactly zero column (no nonzero key) keeps row kk in place
                 const unsigned long long kmax = pkey[kk];
-                const int p = kmax ? 511 - static_cast<int>(kmax & 0x1FFull) : kk;
+                const int p = kmax ? (1 << BITS) - 1 - static_cast<int>(kmax & ((1 << BITS) - 1)) : kk;
                 if (own && pos == p) {
 #pragma unroll
                     for (int j = 0; j < CG; ++j) grow[Q][j] = make_double2(ar[j], ai[j]);
@@ -841,7 +848,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
     if (tid == 0) perm[0] = cnt;
     __syncthreads();
 
-    if (k0 + NB < kf) {
+    if (FUSED && k0 + NB < kf) {
         lu_invert_panel_blocks<NB, true, false>(it, panel, lt_re, lt_im, ut_re, ut_im, tl_re, tl_im, tu_re, tu_im);
         return;
     }
@@ -849,7 +856,7 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
     lu_panel_logdet(it, k0, NB, kf, rsum);
 }
 
-// Panels with more candidate rows than one workgroup holds in registers (lu_rows > LU_MAX_N,
+// Panels with more candidate rows than one workgroup holds in registers (lu_rows > LU_MID_N,
 // up to LU_TALL_MAX): the same factorisation with the panel in global memory (in place; an
 // n x NB panel is a few MB, resident in L2), each thread taking every blockDim-th candidate
 // row.  Per column: pivot search (keys as in pivot_key, 14 position bits), the pivot row
@@ -858,11 +865,6 @@ __global__ __launch_bounds__(LU_MAX_N) void lu_step_kernel(const LuItem* __restr
 // the log-determinant are those of lu_step_kernel.
 constexpr int LU_TALL_MAX = 16383;
 constexpr int LU_TALL_THREADS = 1024;
-
-__device__ __forceinline__ unsigned long long pivot_key_tall(double v, int pos) {
-    return (static_cast<unsigned long long>(__double_as_longlong(v)) & ~0x3FFFull) |
-           static_cast<unsigned long long>(0x3FFF - pos);
-}
 
 template <int NB>
 __global__ __launch_bounds__(LU_TALL_THREADS) void lu_panel_tall_kernel(const LuItem* __restrict__ items, int k0,
@@ -893,7 +895,7 @@ __global__ __launch_bounds__(LU_TALL_THREADS) void lu_panel_tall_kernel(const Lu
         unsigned long long key = 0ull;
         for (int p = kk + tid; p < rows; p += nth) {
             const long o = (long)lu_row(k0, ntop, p) * ld + k0 + kk;
-            const unsigned long long k2 = pivot_key_tall(cabs1(re[o], im[o]), p);
+            const unsigned long long k2 = pivot_key<14>(cabs1(re[o], im[o]), p);
             key = k2 > key ? k2 : key;
         }
         key = wave_max_u64(key);
@@ -1238,9 +1240,7 @@ __global__ __launch_bounds__(LU_UPD_THREADS) void lu_update_kernel(const LuItem*
 }
 
 // Factorise the first kf columns of nitems m x ncols matrices of one shape (identity rows
-// above nt as described at the top; nt = 0 for a general matrix).  Panels with at most
-// LU_MAX_N candidate rows run in registers (lu_step_kernel), larger ones up to LU_TALL_MAX
-// in global memory (lu_panel_tall_kernel).
+// above nt as described at the top; nt = 0 for a general matrix), with up to LU_TALL_MAX candidate rows.
 inline void launch_lu_shape(const LuItem* d_items, int nitems, int m, int ncols, int kf, int nt, int add_identity,
                             hipStream_t s, int nupd = 0) {
     if (kf > ncols || kf > m || (nt > 0 && (kf % LU_NB != 0 || nt > m)))
@@ -1262,7 +1262,7 @@ inline void launch_lu_shape(const LuItem* d_items, int nitems, int m, int ncols,
         const int rows = lu_rows(kp >= 0 ? kp : k0, m, nt);
         // at least 4 waves: the strips and the inversion of L11 and U11 take that many
         const int threads = std::max(256, ((rows + 63) / 64) * 64);
-        hipLaunchKernelGGL(lu_step_kernel<LU_NB>, dim3(units * nitems), dim3(threads), 0, s, d_items, nitems, k0,
+        hipLaunchKernelGGL((lu_step_kernel<LU_NB, LU_MAX_N>), dim3(units * nitems), dim3(threads), 0, s, d_items, nitems, k0,
                            k0 == 0 ? add_identity : 0, kp, cs, strips, defer);
         ISLE_HIP(hipGetLastError());
     };
@@ -1273,9 +1273,13 @@ inline void launch_lu_shape(const LuItem* d_items, int nitems, int m, int ncols,
             kp = k0;
             continue;
         }
-        // the panel in global memory, its elimination on tiles (rows do not grow with k0: none is pending)
-        hipLaunchKernelGGL(lu_panel_tall_kernel<LU_NB>, dim3(nitems), dim3(LU_TALL_THREADS), 0, s, d_items, k0,
-                           k0 == 0 ? add_identity : 0);
+        // the panel alone, its elimination on tiles (rows do not grow with k0: none is pending)
+        if (rows <= LU_MID_N)
+            hipLaunchKernelGGL((lu_step_kernel<LU_NB, LU_MID_N>), dim3(nitems), dim3((rows + 63) / 64 * 64), 0, s, d_items,
+                               nitems, k0, k0 == 0 ? add_identity : 0, -1, 0, 0, 0);
+        else
+            hipLaunchKernelGGL(lu_panel_tall_kernel<LU_NB>, dim3(nitems), dim3(LU_TALL_THREADS), 0, s, d_items, k0,
+                               k0 == 0 ? add_identity : 0);
         ISLE_HIP(hipGetLastError());
         const int ntr = rows - LU_NB, nsw = ncols - k0 - LU_NB;  // columns right of the panel
         const int ntc = nu - k0 - LU_NB;                         // of them updated

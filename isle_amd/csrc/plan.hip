@@ -1524,6 +1524,133 @@ Cyclic add_cyclic_factor(Builder& b, int n, int ng, int nb, PF P, double* logdet
     }
     return c;
 }
+
+// log det of the block-cyclic matrix of the group products (see above) as a tree: a row C x_a + B x_b for
+// every group (C = 1, B = -P_a, b = a + 1; + P in the last), neighbouring rows i (a to b) and j (b to c)
+// merged by eliminating x_b from
+//   W = [[C_j, B_j, 0], [B_i, 0, C_i]]    (columns x_b, x_c, x_a)
+// whose last n rows then are C', B' of the row a to c; the last row closes the cycle with the LU of B + C.
+// Column x_b is zero outside the two rows of W, so the pivots of a merge are those of GEPP on the whole
+// matrix with its columns in this order, and no product of groups is formed; n even makes all block
+// permutations even.  C_j = 1 at the leaves (and for the odd row out): the candidate rows are then few
+// (see lu.hpp).  The merges of a level run together: log2(ng) + 1 factorisations in sequence instead of the ng
+// of add_cyclic_factor.
+// logdet slots: [nb][ng], one per LU.  Requires n % 32 == 0.
+//
+// A merge of two products eliminates 2 n full rows, half again the work of a leaf, so the tree pays while
+// the sequence of panels is the longer part: its time goes like n per factorisation, the work like nb n^3.
+// Sequence -> tree in ms, n = 288: ng = 16: nb = 2 13.1 -> 5.0, 32 26.3 -> 22.1, 48 33.7 -> 32.0, 64 41.8 -> 42.0,
+// 96 60.2 -> 62.0; nb = 32: ng = 8 12.5 -> 11.3, 6 9.15 -> 9.03, 4 5.77 -> 5.90; nb = 2: ng = 4 3.09 -> 2.56, 3
+// 2.30 -> 2.44; n = 128, ng = 8: nb = 96 4.72 -> 4.16, 192 7.39 -> 7.60; n = 384: nb = 8, ng = 16 24.4 -> 15.2,
+// nb = 64, ng = 32 196 -> 190.  n <= 384: the 2 n candidate rows of a merge then fit the registers of a workgroup.
+inline bool tree_logdet(int n, int ng, int nb) {
+    return ng >= 4 && 2 * n <= LU_MID_N && (double)nb * n * n < 331776.0 * ng;
+}
+template <typename PF>
+void add_tree_logdet(Builder& b, int n, int ng, int nb, PF P, double* logdet) {
+    const long nn = (long)n * n, ld = 3L * n, wsz = 2 * 2 * n * ld;  // W: re plane, im plane
+    const size_t lwork = lu_work_doubles(n, (int)ld);
+    // the W of a level are read while the next level's are filled
+    const int most[2] = {ng / 2, (ng - ng / 2) / 2};
+    double* pool[2] = {b.d64((size_t)nb * most[0] * wsz), b.d64((size_t)nb * std::max(most[1], 1) * wsz)};
+    double* work = b.d64((size_t)nb * most[0] * lwork);
+    int* piv = b.di((size_t)nb * most[0] * n);
+    struct Row {
+        int leaf;         // its group, or -1: rows n.. of W number `w` in pool `lv`
+        int lv, w;
+    };
+    auto wmat = [&](int item, int lv, int w) {
+        double* r = pool[lv] + ((long)item * most[lv] + w) * wsz;
+        return CMat<double>{r, r + wsz / 2};
+    };
+    std::vector<Row> rows;
+    for (int j = 0; j < ng; ++j) rows.push_back({j, 0, 0});
+    int slot = 0, lv = 0;
+    const CMat<double> none{nullptr, nullptr};
+    while (rows.size() > 1) {
+        std::vector<Row> merged;
+        std::vector<BlockItem> v;
+        for (int leaf = 1; leaf >= 0; --leaf) {  // merges with C_j = 1, then the general ones
+            std::vector<LuItem> lu;
+            std::vector<TrsmMat> tm;
+            std::vector<GemmItem<double>> gs;
+            v.clear();
+            for (size_t r = 0; r + 1 < rows.size(); r += 2) {
+                const Row &ri = rows[r], &rj = rows[r + 1];
+                if ((rj.leaf >= 0) != (leaf == 1)) continue;
+                const int k = (int)r / 2;
+                for (int item = 0; item < nb; ++item) {
+                    const CMat<double> w = wmat(item, lv, k);
+                    auto put = [&](int row, int col, const CMat<double>& src, long lds, int mode) {
+                        const long o = (long)row * n * ld + (long)col * n;
+                        v.push_back({w.re + o, w.im + o, src.re, src.im, ld, lds, n, n, mode});
+                    };
+                    auto side = [&](const Row& x, int row, int bcol, int ccol) {
+                        if (x.leaf >= 0) {
+                            put(row, bcol, P(item, x.leaf), n, x.leaf == ng - 1 ? 2 : 3);
+                            put(row, ccol, none, 0, 1);
+                        } else {
+                            const CMat<double> m = wmat(item, x.lv, x.w);
+                            const long o = (long)n * ld + n;  // B', then C'
+                            put(row, bcol, {m.re + o, m.im + o}, ld, 2);
+                            put(row, ccol, {m.re + o + n, m.im + o + n}, ld, 2);
+                        }
+                    };
+                    side(rj, 0, 1, 0);
+                    put(0, 2, none, 0, 0);
+                    side(ri, 1, 0, 2);
+                    put(1, 1, none, 0, 0);
+                    const size_t q = (size_t)item * most[0] + k;
+                    LuItem it{w.re, w.im, piv + q * n, logdet + ((long)item * ng + slot + k) * 2, work + q * lwork, n, (int)ld};
+                    it.m = 2 * n;
+                    it.ncols = (int)ld;
+                    it.kf = n;
+                    it.nt = leaf ? n : 0;
+                    it.nupd = n;
+                    lu.push_back(it);
+                    tm.push_back({w.re, w.im, ld, it.work, w.re + n, w.im + n, ld, w.re + n, w.im + n, ld});
+                    GemmItem<double> g{};
+                    g.a_re = w.re + (long)n * ld;  // L21
+                    g.a_im = w.im + (long)n * ld;
+                    g.b_re = w.re + n;  // U12
+                    g.b_im = w.im + n;
+                    g.c_re = w.re + (long)n * ld + n;  // A22
+                    g.c_im = w.im + (long)n * ld + n;
+                    g.m = n;
+                    g.n = 2 * n;
+                    g.k = n;
+                    g.lda = g.ldb = g.ldc = (int)ld;
+                    gs.push_back(g);
+                }
+            }
+            if (lu.empty()) continue;
+            b.add(K::BLOCK, v, 0, 0, 0, (int)nn);
+            b.add(K::LU_SHAPE_DEFER, lu, 2 * n, (int)ld, n, leaf ? n : 0);
+            add_trsm(b, 0, n, 2 * n, tm);
+            b.add(K::GEMM64_CC_SUB, gs, n, 2 * n);
+        }
+        for (size_t r = 0; r < rows.size(); r += 2)
+            merged.push_back(r + 1 < rows.size() ? Row{-1, lv, (int)r / 2} : rows[r]);
+        slot += (int)rows.size() / 2;
+        rows = std::move(merged);
+        lv ^= 1;
+    }
+    double* F = b.d64((size_t)nb * 2 * nn);  // B + C
+    std::vector<BlockItem> v1, v2;
+    std::vector<LuItem> lu;
+    for (int item = 0; item < nb; ++item) {
+        const CMat<double> m = wmat(item, rows[0].lv, rows[0].w);
+        double* f = F + (long)item * 2 * nn;
+        const long o = (long)n * ld + n;
+        v1.push_back({f, f + nn, m.re + o, m.im + o, n, ld, n, n, 2});
+        v2.push_back({f, f + nn, m.re + o + n, m.im + o + n, n, ld, n, n, 4});
+        const size_t q = (size_t)item * most[0];
+        lu.push_back({f, f + nn, piv + q * n, logdet + ((long)item * ng + slot) * 2, work + q * lwork, n, n});
+    }
+    b.add(K::BLOCK, v1, 0, 0, 0, (int)nn);
+    b.add(K::BLOCK, v2, 0, 0, 0, (int)nn);
+    b.add(K::LU, lu, n, 0, 0);
+}
 }  // namespace
 
 // Stable log det M: FP64 group products (as in the grouped form), then the structured
@@ -1547,7 +1674,9 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
     double* ph = b.d64((size_t)nb * 2 * nt * n);
     const bool chains = chain_fits(n);
     double* Wg = b.d64((size_t)nb * ng * (chains ? 1 : 2) * 2 * nn);  // P_j, or two products in turn
-    op->logdet = b.d64((size_t)nb * (ng - 1) * 2);
+    const bool tree = tree_logdet(n, ng, nb);
+    op->slots = tree ? ng : ng - 1;  // log dets per item
+    op->logdet = b.d64((size_t)nb * op->slots * 2);
     auto D = [&](int item, int t) { return CMat<double>{ph + (long)item * 2 * nt * n + (long)t * n,
                                                         ph + (long)item * 2 * nt * n + (long)nt * n + (long)t * n}; };
     auto mW = [&](int item, int j, int k) { return cmat(Wg, ((long)item * ng + j) * 2 + k, nn); };
@@ -1579,7 +1708,10 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
             }
         b.add(K::GEMM64_RC_ROW, gi, n, n);
     }
-    add_cyclic_factor(b, n, ng, nb, P, op->logdet);
+    if (tree)
+        add_tree_logdet(b, n, ng, nb, P, op->logdet);
+    else
+        add_cyclic_factor(b, n, ng, nb, P, op->logdet);
     b.finish();
     tune(*op);
     auto& ref = *op;
@@ -1901,8 +2033,7 @@ void Plan::logdetM(const double* phi, int nt, int batch, int mode, int group, in
     OpCache& op = mode == 0   ? get_logdet_plain(nt, batch, nspecies, spin)
                   : mode == 1 ? get_logdet_grouped(nt, batch, group, nspecies, spin)
                               : get_logdet_stable(nt, batch, group, nspecies, spin);
-    // log-determinant slots per (field, species): one, or one per elimination step
-    const int per = (mode == 2 && nt / group > 1) ? nt / group - 1 : 1;
+    const int per = op.slots;
     run(op, phi);
     // sums of phi per field
     DevBuf sums((size_t)batch * 4 * 8);

@@ -99,7 +99,8 @@ struct OpCache {
     std::vector<char> blob;    // host copy of the descriptors (for merged operations)
     std::vector<double*> extra;  // operation-specific result buffers (the QLU blocks)
     long phi_stride = 0;       // doubles between consecutive fields of the batch
-    double* logdet = nullptr;  // device [batch][nspecies][2]
+    double* logdet = nullptr;  // device [batch][nspecies][slots][2]
+    int slots = 1;             // log dets whose sum is an item's (one per elimination step)
     double* parts = nullptr;   // device [batch][nspecies][nx*nt] interleaved
     bool direct = false;       // the last step (DREDUCE) writes the parts to the caller's array
     int nspecies = 0;
