@@ -232,7 +232,8 @@ void add_trsm(Builder& b, int mode, int n, int w, const std::vector<TrsmMat>& ma
 //   GL_{ng-1} = I, GL_j = P_{j+1} GL_{j+1};  Mid = (1 + P_0 GL_0)^{-1}
 //   RR_0 = Mid, RR_j = RR_{j-1} P_{j-1};     K_j = GL_j RR_j
 // trsm: the inverse by blocked triangular solves on GEMMs (n % 32 == 0; many matrices), else by
-// lu_solve_kernel (few: one launch instead of four per pair of panels).
+// lu_solve_kernel (few: one launch instead of four per pair of panels).  keep: P_0 is read again afterwards;
+// with a single group it is otherwise factorised in place.
 struct TopLevel {
     double *KK, *RR;
     int ng;
@@ -242,26 +243,25 @@ struct TopLevel {
     }
 };
 template <typename PF>
-TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm) {
+TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm, bool keep) {
     const long nn = (long)n * n;
     double* GL = b.d64((size_t)nb * ng * 2 * nn);
     double* RR = b.d64((size_t)nb * ng * 2 * nn);
     double* KK = b.d64((size_t)nb * ng * 2 * nn);
-    double* LUb = b.d64((size_t)nb * 2 * nn);
+    double* LUb = ng > 1 || keep ? b.d64((size_t)nb * 2 * nn) : nullptr;
+    auto fac = [&](int item) { return LUb ? cmat(LUb, item, nn) : mP(item, 0); };
     int* piv = b.di((size_t)nb * n);
     auto m64 = [&](double* base, int item, int j) { return cmat(base, (long)item * ng + j, nn); };
-    if (ng == 1) {
+    auto gl = [&](int item, int j) { return j == ng - 2 ? mP(item, ng - 1) : m64(GL, item, j); };
+    if (ng == 1 && keep) {
         std::vector<CopyItem<double, double>> cp;
         for (int item = 0; item < nb; ++item) cp.push_back({mP(item, 0).re, LUb + (long)item * 2 * nn, 2 * nn});
         b.add(K::COPY64, cp, (int)(2 * nn));
-    } else {
-        std::vector<CopyItem<double, double>> cp;
-        for (int item = 0; item < nb; ++item) cp.push_back({mP(item, ng - 1).re, m64(GL, item, ng - 2).re, 2 * nn});
-        b.add(K::COPY64, cp, (int)(2 * nn));
+    } else if (ng > 1) {
         for (int j = ng - 3; j >= 0; --j) {
             std::vector<GemmItem<double>> gi;
             for (int item = 0; item < nb; ++item) {
-                const CMat<double> a = mP(item, j + 1), bb = m64(GL, item, j + 1);
+                const CMat<double> a = mP(item, j + 1), bb = gl(item, j + 1);
                 gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(GL, item, j), nullptr, nullptr, nullptr,
                                            nullptr, n));
             }
@@ -269,7 +269,7 @@ TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm) {
         }
         std::vector<GemmItem<double>> gi;
         for (int item = 0; item < nb; ++item) {
-            const CMat<double> a = mP(item, 0), bb = m64(GL, item, 0);
+            const CMat<double> a = mP(item, 0), bb = gl(item, 0);
             gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, cmat(LUb, item, nn), nullptr, nullptr, nullptr,
                                        nullptr, n));
         }
@@ -279,7 +279,7 @@ TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm) {
         std::vector<LuItem> lu;
         double* luw = b.d64(nb * lu_work_doubles(n));
         for (int item = 0; item < nb; ++item)
-            lu.push_back({LUb + (long)item * 2 * nn, LUb + (long)item * 2 * nn + nn, piv + (long)item * n, nullptr,
+            lu.push_back({fac(item).re, fac(item).im, piv + (long)item * n, nullptr,
                           luw + item * lu_work_doubles(n), n, n});
         b.add(K::LU, lu, n, 0, 1);
         if (trsm) {
@@ -293,7 +293,7 @@ TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm) {
             std::vector<TrsmMat> tl, tu;
             for (int item = 0; item < nb; ++item) {
                 const CMat<double> s1 = cmat(S1, item, nn), s2 = cmat(S2, item, nn), rr = m64(RR, item, 0);
-                const double* fre = LUb + (long)item * 2 * nn;
+                const double* fre = fac(item).re;
                 sv.push_back({piv + (long)item * n, sig + (long)item * n, n, n});
                 ga.push_back({sig + (long)item * n, nullptr, nullptr, s1.re, s1.im, nullptr, nullptr, n, n, n, n, 0});
                 tl.push_back({fre, fre + nn, n, luw + item * lu_work_doubles(n), s1.re, s1.im, n, s2.re, s2.im, n});
@@ -307,7 +307,7 @@ TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm) {
             std::vector<SolveItem> sv;
             for (int item = 0; item < nb; ++item) {
                 SolveItem si{};
-                si.lu_re = LUb + (long)item * 2 * nn;
+                si.lu_re = fac(item).re;
                 si.lu_im = si.lu_re + nn;
                 si.piv = piv + (long)item * n;
                 si.dinv = luw + item * lu_work_doubles(n);
@@ -335,7 +335,7 @@ TopLevel add_top_level(Builder& b, int n, int ng, int nb, PF mP, bool trsm) {
         std::vector<GemmItem<double>> gi;
         for (int item = 0; item < nb; ++item)
             for (int j = 0; j < ng - 1; ++j) {
-                const CMat<double> a = m64(GL, item, j), bb = m64(RR, item, j);
+                const CMat<double> a = gl(item, j), bb = m64(RR, item, j);
                 gi.push_back(gitem<double>(a.re, a.im, bb.re, bb.im, m64(KK, item, j), nullptr, nullptr, nullptr,
                                            nullptr, n));
             }
@@ -1026,7 +1026,7 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
         b.add(K::GEMM64_RC_ROW, gi, n, n);
     }
     // ---- top level (FP64)
-    const TopLevel tl = add_top_level(b, n, ng, nb, mP, n % LU_NB == 0);
+    const TopLevel tl = add_top_level(b, n, ng, nb, mP, n % LU_NB == 0, true);
     // ---- local right chains (FP32), transposed.  With n % 32 == 0 the chain products also
     //      produce the force diagonal f[tau] = rowdot(Suf_{tau+1}, Rt_tau) (diag Rt at a group's
     //      last slice) as partial row sums per 16 columns, summed by one reduction at the end,
@@ -1164,7 +1164,7 @@ OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin
     b.add(K::PHASE, phs);
     add_suffix(b, nt, g, nb, nspecies, ph, [&](int item, int j) { return mS(item, j * g + g - 1).re; }, -2 * nn, 1);
     const TopLevel tl = add_top_level(b, n, ng, nb, [&](int item, int j) { return mS(item, j * g); },
-                                      n % LU_NB == 0 && nb > 4);
+                                      n % LU_NB == 0 && nb > 4, false);
     add_right(b, *op, nt, g, nb, nspecies, ph, ph32, Suf, [&](int item, int j) { return ChainK{tl.k(item, j), nn, n, 1.0}; });
     b.finish();
     tune(*op);
