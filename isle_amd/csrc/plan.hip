@@ -532,6 +532,8 @@ void Plan::run(OpCache& op, const double* phi, double* out) {
         if (!launch_step(op, st, phi, out)) throw std::runtime_error("a step's launch shape does not fit it");
 }
 
+static std::tuple<int, int, int, int> tune_key(const Step& st);
+
 void Plan::set_tile(int kind, int tile) {
     if (kind < 0 || kind >= (int)K::KIND_END) throw std::invalid_argument("unknown step kind");
     if (tile < -1 || tile >= N_TILES) throw std::invalid_argument("tile out of range");
@@ -545,7 +547,7 @@ void Plan::set_tile(int kind, int tile) {
             if (tile >= 0) {
                 st.tile = tile;
             } else {
-                auto f = tuned_.find(std::make_tuple((int)st.kind, st.max_m, st.max_n, st.count));
+                auto f = tuned_.find(tune_key(st));
                 if (f != tuned_.end()) st.tile = f->second;
             }
         }
@@ -563,6 +565,17 @@ static bool is_gemm(K k) {
            k == K::GEMM64_CC4_SUB;
 }
 
+// Products that a launch shape is timed on: with more than eight rounds of 64 x 64 tiles on every CU the
+// count decides no longer, and operations of several such counts share one choice (the tree of the stable
+// log det, n = 288, 32 matrices: first pass 79 ms against 215 with each count timed whole).
+static int tune_count(const Step& st) {
+    const double tiles = (double)st.max_m * st.max_n / (64.0 * 64.0);
+    return std::min(st.count, std::max(1, (int)std::ceil(8.0 * CHAIN_CUS / std::max(tiles, 1e-3))));
+}
+static std::tuple<int, int, int, int> tune_key(const Step& st) {
+    return std::make_tuple((int)st.kind, st.max_m, st.max_n, tune_count(st));
+}
+
 void Plan::tune(OpCache& op) {
     hipEvent_t e0, e1;
     ISLE_HIP(hipEventCreate(&e0));
@@ -574,7 +587,7 @@ void Plan::tune(OpCache& op) {
             st.tile = pinned->second;
             continue;
         }
-        auto key = std::make_tuple((int)st.kind, st.max_m, st.max_n, st.count);
+        auto key = tune_key(st);
         auto f = tuned_.find(key);
         if (f != tuned_.end()) {
             st.tile = f->second;
@@ -582,15 +595,21 @@ void Plan::tune(OpCache& op) {
         }
         float best = 1e30f;
         int best_tile = 0;
-        for (int tile = 0; tile < N_TILES; ++tile) {
-            st.tile = tile;
-            if (!launch_step(op, st, nullptr)) continue;  // shape does not fit; warm up otherwise
+        Step probe = st;
+        probe.count = tune_count(st);
+        auto timed = [&](int reps) {
             ISLE_HIP(hipEventRecord(e0, stream_));
-            for (int r = 0; r < 3; ++r) launch_step(op, st, nullptr);
+            for (int r = 0; r < reps; ++r) launch_step(op, probe, nullptr);
             ISLE_HIP(hipEventRecord(e1, stream_));
             ISLE_HIP(hipEventSynchronize(e1));
             float ms = 0;
             ISLE_HIP(hipEventElapsedTime(&ms, e0, e1));
+            return ms / reps;
+        };
+        for (int tile = 0; tile < N_TILES; ++tile) {
+            probe.tile = tile;
+            if (!launch_step(op, probe, nullptr)) continue;  // shape does not fit; warm up otherwise
+            const float ms = timed(3);
             if (ms < best) {
                 best = ms;
                 best_tile = tile;
