@@ -168,7 +168,7 @@ def config4(args):
 # the dominant kind's kernel as it appears in the rocprofv3 PMC summary of this workload
 PMC_SUMMARY = "profiles/force_mixed_nx288_nt128_chains128_hbm_traffic.md"
 PMC_CHAINS = 128
-PMC_ROWS = {"gemm64_rc_row": ("gemm_rcd_kernel<double, 1, false, 96, 96, 16, 2, 2, 6>", "7077888")}
+PMC_ROWS = {"suffix64_chains": ("suffix_chain_kernel<3, 0, 2>", "7077888")}
 
 
 def _pmc_traffic(kind, chains):
