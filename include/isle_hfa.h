@@ -87,7 +87,8 @@ int isle_logdetM_batch(isle_hfm* h, const double* phi, int nt, int batch, int mo
 /* forceDirectSinglePart(hfm, phi, K, species) for each species (without the -i factor)
  *   src/isle/cpp/action/hubbardFermiAction.cpp:16-60.
  * mode 0: plain FP64 reference algorithm; mode 1: FP32 chains over groups of `group`
- * slices on MFMA with an FP64 combination of the group products; mode 2: FP64 chains over
+ * slices (the most; fewer where few fields leave the GPU idle) on MFMA with an FP64 combination
+ * of the group products; mode 2: FP64 chains over
  * the groups with the combination taken from the elimination of mode 2 of logdetM_batch
  * (same size limits); mode 3: mode 2 with the right chains in FP32 on MFMA (two groups or
  * more).

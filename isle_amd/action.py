@@ -8,10 +8,13 @@ Besides the reference's single-field ``eval``/``force``, HubbardFermiAction offe
 ``eval_batch``/``force_batch`` over a [batch, nx*nt] tensor of independent fields, and a
 ``precision`` switch:
 
-* ``"fp64"``  - the reference DIRECT_SINGLE algorithm, every product in FP64;
-* ``"mixed"`` - force from FP32 chains over groups of ``group`` time slices on MFMA,
-  combined in FP64; eval (the Metropolis action) from FP64 group products, multiplied
-  together (``logdet="grouped"``) or combined through the stabilising block-cyclic LU with
+* ``"fp64"``  - the reference DIRECT_SINGLE algorithm, every product in FP64.  Where few fields would leave
+  the GPU idle (Nx > 128), the chains of time slices are cut into groups that run side by side; the number
+  of groups depends on the number of fields in the call, so a field's result depends in its last bits on
+  the batch that it is evaluated in;
+* ``"mixed"`` - force from FP32 chains over groups of at most ``group`` time slices on MFMA
+  (fewer for few fields, as in ``"fp64"``), combined in FP64; eval (the Metropolis action)
+  from FP64 group products, multiplied together (``logdet="grouped"``) or combined through the stabilising block-cyclic LU with
   groups of ``logdet_group`` slices (``logdet="stable"``, default 8).  With
   ``recompute=k`` (k dividing ``group``, Nx a multiple of 32) the force keeps the FP64
   suffix chains only every k slices and recomputes the others when they are needed:

@@ -475,18 +475,26 @@ void Plan::slice_matrix(int species, int inv, double* out_host) {
     ISLE_HIP(hipMemcpy(out_host, src.p, nn * 8, hipMemcpyDeviceToHost));
 }
 
+// Slices of ng groups: group j is slices at[j] .. at[j + 1] - 1, all of nt / ng or one more (those first).
+static std::vector<int> group_starts(int nt, int ng) {
+    std::vector<int> at;
+    for (int j = 0; j <= ng; ++j) at.push_back(j * (nt / ng) + std::min(j, nt % ng));
+    return at;
+}
+
 // Suffix chains of all groups of all (field, species) items in one launch: S_e at out(item, j),
 // the next ones `step` doubles further each (all = 1), or only S_s (all = 0).
 template <typename OF>
-void Plan::add_suffix(Builder& b, int nt, int g, int nb, int nspecies, const double* ph, OF out, long step, int all) {
-    const int n = nx_;
+void Plan::add_suffix(Builder& b, const std::vector<int>& at, int nb, int nspecies, const double* ph, OF out,
+                      long step, int all) {
+    const int n = nx_, nt = at.back();
     std::vector<SuffixItem> v;
     for (int item = 0; item < nb; ++item)
-        for (int j = 0; j < nt / g; ++j) {
+        for (size_t j = 0; j + 1 < at.size(); ++j) {
             const double* d = ph + (long)item * 2 * nt * n;
             const int s = item % nspecies;
-            v.push_back({pk64_[s]->as<double>(), a64_[s]->as<double>(), d, d + (long)nt * n, out(item, j), step,
-                         j * g + g - 1, -1, g, all, 0});
+            v.push_back({pk64_[s]->as<double>(), a64_[s]->as<double>(), d, d + (long)nt * n, out(item, (int)j), step,
+                         at[j + 1] - 1, -1, at[j + 1] - at[j], all, 0});
         }
     b.add(K::SUFFIX64, v, n, n);
 }
@@ -494,23 +502,24 @@ void Plan::add_suffix(Builder& b, int nt, int g, int nb, int nspecies, const dou
 // Right chains of all groups in one launch (FP32 with ph32, else FP64), their force diagonal summed
 // over the strips into the parts; Suf: nt matrices per item.
 template <typename KF>
-void Plan::add_right(Builder& b, OpCache& op, int nt, int g, int nb, int nspecies, const double* ph,
+void Plan::add_right(Builder& b, OpCache& op, const std::vector<int>& at, int nb, int nspecies, const double* ph,
                      const float* ph32, const double* Suf, KF kf) {
-    const int n = nx_, slots = chain_tiles(n);
+    const int n = nx_, nt = at.back(), slots = chain_tiles(n);
     const long nn = (long)n * n;
     double* part = b.d64((size_t)nb * nt * slots * n * 2);
     auto fill = [&](auto* phases, const auto& packed, K kind) {
         typedef std::remove_const_t<std::remove_pointer_t<decltype(phases)>> T;
         std::vector<RightItem<T>> v;
         for (int item = 0; item < nb; ++item)
-            for (int j = 0; j < nt / g; ++j) {
-                const ChainK k = kf(item, j);
-                const double* d0 = ph + (long)item * 2 * nt * n + (long)j * g * n;
+            for (size_t j = 0; j + 1 < at.size(); ++j) {
+                const ChainK k = kf(item, (int)j);
+                const int s = at[j], g = at[j + 1] - s;
+                const double* d0 = ph + (long)item * 2 * nt * n + (long)s * n;
                 const T* d = phases + (long)item * 2 * nt * n;
                 v.push_back({packed[item % nspecies]->template as<T>(), k.re, k.re + k.plane, k.ld, k.sign, d0,
                              d0 + (long)nt * n, d, d + (long)nt * n,
-                             g > 1 ? Suf + ((long)item * nt + j * g + 1) * 2 * nn : nullptr, 2 * nn,
-                             part + ((long)item * nt + j * g) * slots * n * 2, j * g, g});
+                             g > 1 ? Suf + ((long)item * nt + s + 1) * 2 * nn : nullptr, 2 * nn,
+                             part + ((long)item * nt + s) * slots * n * 2, s, g});
             }
         b.add(kind, v, n, n);
     };
@@ -1154,10 +1163,12 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
 
 // The grouped force on the strip kernels (chain.hpp): every group's suffix chain in one launch,
 // the top level, every group's right chain with the diagonal fused in one launch.  right32: the
-// mixed form (FP32 right chains); else FP64 throughout.
-OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin, bool right32) {
+// mixed form (FP32 right chains); else FP64 throughout.  g: most slices of a group (chain_groups may
+// take shorter ones); items: (field, species) pairs that share the launches, 0 for this batch's alone.
+OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin, bool right32, int items) {
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
-    auto key = std::make_tuple(right32 ? 1 : 0, nt, batch, g, nspecies, spin);
+    const int ng = chain_groups(nt, items > 0 ? items : batch * nspecies, nt / g, right32 ? MIXED : PLAIN);
+    auto key = std::make_tuple(right32 ? 1 : 0, nt, batch, g, nspecies, spin + 2 * ng);
     auto found = cache_.find(key);
     if (found != cache_.end()) return *found->second;
     auto op = std::make_unique<OpCache>();
@@ -1166,7 +1177,8 @@ OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin
     op->nspecies = nspecies;
     op->phi_stride = 2L * nx_ * nt;
     Builder b(*op);
-    const int n = nx_, nb = batch * nspecies, ng = nt / g;
+    const int n = nx_, nb = batch * nspecies;
+    const std::vector<int> at = group_starts(nt, ng);
     const long nn = (long)n * n;
     double* ph = b.d64((size_t)nb * 2 * nt * n);
     float* ph32 = right32 ? b.d32((size_t)nb * 2 * nt * n) : nullptr;
@@ -1181,10 +1193,10 @@ OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin
                        right32 ? d32 + (long)nt * n : nullptr, n, nt});
     }
     b.add(K::PHASE, phs);
-    add_suffix(b, nt, g, nb, nspecies, ph, [&](int item, int j) { return mS(item, j * g + g - 1).re; }, -2 * nn, 1);
-    const TopLevel tl = add_top_level(b, n, ng, nb, [&](int item, int j) { return mS(item, j * g); },
+    add_suffix(b, at, nb, nspecies, ph, [&](int item, int j) { return mS(item, at[j + 1] - 1).re; }, -2 * nn, 1);
+    const TopLevel tl = add_top_level(b, n, ng, nb, [&](int item, int j) { return mS(item, at[j]); },
                                       n % LU_NB == 0 && nb > 4, false);
-    add_right(b, *op, nt, g, nb, nspecies, ph, ph32, Suf, [&](int item, int j) { return ChainK{tl.k(item, j), nn, n, 1.0}; });
+    add_right(b, *op, at, nb, nspecies, ph, ph32, Suf, [&](int item, int j) { return ChainK{tl.k(item, j), nn, n, 1.0}; });
     b.finish();
     tune(*op);
     auto& ref = *op;
@@ -1707,7 +1719,8 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
     auto P = [&](int item, int j) {
         return chains ? cmat(Wg, (long)item * ng + j, nn) : mW(item, j, (g - 1) & 1);
     };
-    if (chains) add_suffix(b, nt, g, nb, nspecies, ph, [&](int item, int j) { return P(item, j).re; }, 0, 0);
+    if (chains)
+        add_suffix(b, group_starts(nt, ng), nb, nspecies, ph, [&](int item, int j) { return P(item, j).re; }, 0, 0);
     std::vector<ScaleItem<double>> sc;
     for (int item = 0; item < nb && !chains; ++item)
         for (int j = 0; j < ng; ++j) {
@@ -1748,6 +1761,8 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
 OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin, bool right32) {
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
     if (right32 && nt / g < 2) throw std::invalid_argument("FP32 right chains of the stable force need two groups or more");
+    // a single group is the plain form: nothing to eliminate
+    if (nt == g && chain_fits(nx_)) return get_force_chains(nt, batch, nt, nspecies, spin, false, 0);
     auto key = std::make_tuple(right32 ? 6 : 4, nt, batch, g, nspecies, spin);
     auto found = cache_.find(key);
     if (found != cache_.end()) return *found->second;
@@ -1768,7 +1783,7 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
     const bool chains = chain_fits(n);
     double* Rt = right32 || chains ? nullptr : b.d64((size_t)nb * nt * 2 * nn);
     float* Rt32 = right32 && !chains ? b.d32((size_t)nb * ng * 2 * 2 * nn) : nullptr;  // last two products per group
-    double* Kt = right32 || (chains && ng > 1) ? nullptr : b.d64((size_t)nb * ng * 2 * nn);
+    double* Kt = right32 || chains ? nullptr : b.d64((size_t)nb * ng * 2 * nn);
     float* K32 = right32 && !chains ? b.d32((size_t)nb * ng * 2 * nn) : nullptr;
     double* Tb = b.d64((size_t)nb * ng * 2 * n * wd);
     op->parts = b.d64((size_t)nb * nt * n * 2);
@@ -1793,7 +1808,8 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
                        right32 ? D32(item, 0).re : nullptr, right32 ? D32(item, 0).im : nullptr, n, nt});
     b.add(K::PHASE, phs);
     if (chains)
-        add_suffix(b, nt, g, nb, nspecies, ph, [&](int item, int j) { return mS(item, j * g + g - 1).re; }, -2 * nn, 1);
+        add_suffix(b, group_starts(nt, ng), nb, nspecies, ph,
+                   [&](int item, int j) { return mS(item, j * g + g - 1).re; }, -2 * nn, 1);
     if (!chains) {
         std::vector<ScaleItem<double>> sc;
         for (int item = 0; item < nb; ++item)
@@ -1852,8 +1868,8 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
             si.dinv = luw + item * lu_work_doubles(n);
             si.x_re = mK(item, 0).re;
             si.x_im = mK(item, 0).im;
-            si.xsr = chains ? n : 1;  // K, or K^T for the chain products
-            si.xsc = chains ? 1 : n;
+            si.xsr = 1;  // written transposed: K^T
+            si.xsc = n;
             si.n = n;
             si.ld = n;
             si.nrhs = n;
@@ -1965,8 +1981,7 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
         }
     }
     if (chains) {
-        add_right(b, *op, nt, g, nb, nspecies, ph, ph32, Suf, [&](int item, int j) {
-            if (ng == 1) return ChainK{mK(item, 0).re, nn, n, 1.0};
+        add_right(b, *op, group_starts(nt, ng), nb, nspecies, ph, ph32, Suf, [&](int item, int j) {
             const CMat<double> x = j < ng - 1 ? mT(item, j + 1) : mT(item, 0);
             return ChainK{x.re + (j < ng - 1 ? (long)(j + 1) * n : 0), (long)n * wd, wd, j < ng - 1 ? -1.0 : 1.0};
         });
@@ -2086,37 +2101,44 @@ void Plan::logdetM(const double* phi, int nt, int batch, int mode, int group, in
     }
 }
 
-// Slices per group of the plain FP64 force for nb (field, species) items: one chain over all
-// slices (the reference's own order of products), or, for lattices beyond the register-resident
-// strip kernels (n > CHAIN_MAX_RES), the grouping with the shortest time where few items leave the
-// GPU idle.  Times in MFMA cycles of a SIMD: a slice takes its tiles' products (32 n each) and
-// about 900 cycles of latency, a top-level product (2 ng - 1 of them in sequence) about 7000 cycles
-// and its share of n^3.  One field at n = 288, Nt = 96: 6.4 ms with one group, 2.06 ms with six.
-int Plan::plain_group(int nt, int nb) const {
+// Groups of the strip chains of nb (field, species) items, at least `least` of them: that many, or, for
+// n > CHAIN_MAX_RES, the number with the shortest time where few items leave the GPU idle.  The result is
+// as accurate either way (ten fields each, n = 144 .. 384, Nt 31 .. 97: errors against 64 bits 0.8 to 1.3 of
+// one chain's), but rounded differently, so an item's last bits depend on nb.  Up to CHAIN_MAX_RES a slice
+// takes 3 us and grouping gave 4% of a gradient at n = 72, not worth an order of products other than the
+// reference's.  Times in MFMA cycles of a SIMD: a slice takes its tiles' products (32 n each) and about 900
+// cycles of latency (0.6 of both in FP32); a product of two groups takes its 64 x 64 tiles in rounds over
+// the CUs, 200 n each, and about 10000 to start; the force has 2 ng - 2 of those in sequence and one of all
+// K_j.  One field, one group -> this choice, in ms (a launch per slice where the strips are not used):
+//   FP64 force    n = 288, Nt 97: 5.65 -> 1.85 (3.33)   n = 384: 7.93 -> 3.00 (5.57)   n = 512: 13.5 -> 5.49 (7.69)
+//   mixed force   n = 288, Nt 32: 1.97 -> 1.23 (2.01)   n = 384: 2.85 -> 1.85 (2.75)   n = 512: 4.70 -> 3.00 (3.67)
+// and with four fields of 32 slices one group at n = 384 (FP64 3.43; four groups 3.72) and 512.
+int Plan::chain_groups(int nt, int nb, int least, ChainUse what) {
     const int n = nx_, tiles = chain_tiles(n);
-    if (n <= CHAIN_MAX_RES) return nt;
-    int best = nt;
+    if (n <= CHAIN_MAX_RES) return least;
+    int& best = groups_[std::make_tuple(nt, nb, least, (int)what)];
+    if (best > 0) return best;
+    const long t64 = (long)cdiv(n, 64) * cdiv(n, 64);
+    auto product = [&](long items) { return 10000.0 + 200.0 * n * ((items * t64 + CHAIN_CUS - 1) / CHAIN_CUS); };
     double cost = 0;
-    for (int ng = 1; ng <= std::max(1, nt / 4); ++ng) {
-        if (nt % ng != 0) continue;
-        const long t1 =
-            chain_cost(CHAIN_SHAPES[chain_shape<double>(n, nb * ng, CHAIN_CUS)], tiles, nb * ng, CHAIN_CUS);
-        const double slice = t1 * 32.0 * n * 1.15 + 900.0;
-        const double product = 7000.0 + 0.0016 * n * (double)n * n * std::max(1.0, nb / 8.0);
-        const double c = 2.0 * (nt / ng) * slice + (ng > 1 ? (2 * ng - 1) * product : 0.0);
-        if (ng == 1 || c < 0.95 * cost) {
+    for (int ng = least; ng <= std::max(least, nt / 4); ++ng) {
+        const int sh = chain_shape<double>(n, nb * ng, CHAIN_CUS), len = (nt + ng - 1) / ng;
+        const double slice = chain_cost(CHAIN_SHAPES[sh], tiles, nb * ng, CHAIN_CUS) * 32.0 * n * 1.15 + 900.0;
+        double c = (what == MIXED ? 1.6 : 2.0) * len * slice;
+        if (ng > 1) c += (2 * ng - 2) * product(nb) + product((long)nb * (ng - 1));
+        if (ng == least || c < 0.95 * cost) {
             cost = c;
-            best = nt / ng;
+            best = ng;
         }
     }
     return best;
 }
 
-OpCache& Plan::get_force(int mode, int nt, int batch, int group, int nspecies, int spin) {
+OpCache& Plan::get_force(int mode, int nt, int batch, int group, int nspecies, int spin, int items) {
     if (nt < 2) throw std::invalid_argument("nt < 2 in HubbardFermiAction algorithm DIRECT_SINGLE not supported");
     if (chain_fits(nx_)) {
-        if (mode == 0) return get_force_chains(nt, batch, plain_group(nt, batch * nspecies), nspecies, spin, false);
-        if (mode == 1 && !recomputes(group)) return get_force_chains(nt, batch, group, nspecies, spin, true);
+        if (mode == 0) return get_force_chains(nt, batch, nt, nspecies, spin, false, items);
+        if (mode == 1 && !recomputes(group)) return get_force_chains(nt, batch, group, nspecies, spin, true, items);
     }
     return mode == 0   ? get_force_plain(nt, batch, nspecies, spin)
            : mode == 1 ? get_force_mixed(nt, batch, group, nspecies, spin)
@@ -2251,8 +2273,10 @@ void Plan::force_parts_multi(int nops, const double* const* phis, const int* nts
     MultiOp* mo = nullptr;
     if (found == multi_.end()) {
         std::vector<OpCache*> ops;
+        int items = 0;  // the batches share their launches
+        for (int i = 0; i < nops; ++i) items += batches[i] * nspecies;
         for (int i = 0; i < nops; ++i) {
-            OpCache* op = &get_force(mode, nts[i], batches[i], groups[i], nspecies, spin);
+            OpCache* op = &get_force(mode, nts[i], batches[i], groups[i], nspecies, spin, items);
             for (OpCache* o : ops)
                 if (o == op) throw std::invalid_argument("two batches of one shape: join them into one batch");
             ops.push_back(op);

@@ -230,13 +230,16 @@ private:
     bool recomputes(int g) const {
         return recompute_ > 0 && recompute_ < g && g % recompute_ == 0 && nx_ % 32 == 0;
     }
-    int plain_group(int nt, int nb) const;
+    enum ChainUse { PLAIN, MIXED };  // force in FP64, force with FP32 right chains
+    std::map<std::tuple<int, int, int, int>, int> groups_;  // chain_groups' answers
+    int chain_groups(int nt, int nb, int least, ChainUse what);
     template <typename OF>
-    void add_suffix(Builder& b, int nt, int g, int nb, int nspecies, const double* ph, OF out, long step, int all);
+    void add_suffix(Builder& b, const std::vector<int>& at, int nb, int nspecies, const double* ph, OF out, long step,
+                    int all);
     template <typename KF>
-    void add_right(Builder& b, OpCache& op, int nt, int g, int nb, int nspecies, const double* ph, const float* ph32,
-                   const double* Suf, KF kf);
-    OpCache& get_force_chains(int nt, int batch, int group, int nspecies, int spin, bool right32);
+    void add_right(Builder& b, OpCache& op, const std::vector<int>& at, int nb, int nspecies, const double* ph,
+                   const float* ph32, const double* Suf, KF kf);
+    OpCache& get_force_chains(int nt, int batch, int group, int nspecies, int spin, bool right32, int items);
     OpCache& get_logdet_plain(int nt, int batch, int nspecies, int spin);
     OpCache& get_logdet_chains(int nt, int batch, int g, int nspecies, int spin, bool reference);
     OpCache& get_logdet_grouped(int nt, int batch, int group, int nspecies, int spin);
@@ -263,7 +266,7 @@ private:
         std::vector<OpCache*> ops;
     };
     std::map<std::vector<long>, std::unique_ptr<MultiOp>> multi_;
-    OpCache& get_force(int mode, int nt, int batch, int group, int nspecies, int spin);
+    OpCache& get_force(int mode, int nt, int batch, int group, int nspecies, int spin, int items = 0);
     std::unique_ptr<MultiOp> merge_ops(const std::vector<OpCache*>& ops);
 };
 
