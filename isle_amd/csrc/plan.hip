@@ -1360,10 +1360,10 @@ OpCache& Plan::get_logdet_grouped(int nt, int batch, int g, int nspecies, int sp
     return ref;
 }
 
-// log det M on the strip kernels: the products of groups of g slices in one launch, multiplied
+// log det M on the strip kernels: the products of groups of slices in one launch, multiplied
 // together pairwise (all pairs of a level in one launch), then the LU of 1 + (.).  reference: the
-// chains of the reference's algorithm in its order (see get_logdet_plain); else the inverse form
-// X_0 ... X_{nt-1} for both species.
+// chains of the reference's algorithm in its order (see get_logdet_plain), pairs by four real products;
+// else the inverse form X_0 ... X_{nt-1} for both species.  g: most slices of a group.
 OpCache& Plan::get_logdet_chains(int nt, int batch, int g, int nspecies, int spin, bool reference) {
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
     auto key = std::make_tuple(reference ? 2 : 3, nt, batch, g, nspecies, spin);
@@ -1375,12 +1375,14 @@ OpCache& Plan::get_logdet_chains(int nt, int batch, int g, int nspecies, int spi
     op->nspecies = nspecies;
     op->phi_stride = 2L * nx_ * nt;
     Builder b(*op);
-    const int n = nx_, nb = batch * nspecies, ng = nt / g;
+    const int n = nx_, nb = batch * nspecies, ng = chain_groups(nt, nb, nt / g, LOGDET);
+    const std::vector<int> at = group_starts(nt, ng);
     const long nn = (long)n * n;
     double* ph = b.d64((size_t)nb * 2 * nt * n);
-    double* W[2] = {b.d64((size_t)nb * ng * 2 * nn), ng > 1 ? b.d64((size_t)nb * ((ng + 1) / 2) * 2 * nn) : nullptr};
+    double* W = b.d64((size_t)nb * (2 * ng - 1) * 2 * nn);  // the groups' products, then those of the levels
     int* piv = b.di((size_t)nb * n);
     op->logdet = b.d64((size_t)nb * 2);
+    auto mW = [&](int item, int q) { return cmat(W, (long)item * (2 * ng - 1) + q, nn); };
     auto bchain = [&](int item) { return reference && hop_ == EXP && item % nspecies == PARTICLE; };
     std::vector<PhaseItem> phs;
     std::vector<SuffixItem> sv;
@@ -1391,32 +1393,32 @@ OpCache& Plan::get_logdet_chains(int nt, int batch, int g, int nspecies, int spi
         phs.push_back({item / nspecies, spin, fw ? 1.0 : sigma_of(s), d, d + (long)nt * n, nullptr, nullptr, n, nt});
         for (int j = 0; j < ng; ++j)
             sv.push_back({(fw ? pke64_ : pk64_[s])->as<double>(), (fw ? e64_[s] : a64_[s])->as<double>(), d,
-                          d + (long)nt * n, cmat(W[0], (long)item * ng + j, nn).re, 0,
-                          reference ? j * g : j * g + g - 1, reference ? 1 : -1, g, 0, reference});
+                          d + (long)nt * n, mW(item, j).re, 0, reference ? at[j] : at[j + 1] - 1, reference ? 1 : -1,
+                          at[j + 1] - at[j], 0, reference});
     }
     b.add(K::PHASE, phs);
     b.add(K::SUFFIX64, sv, n, n);
-    int k = ng, at = 0;  // k products per item, in W[at]
-    for (; k > 1; k = (k + 1) / 2, at ^= 1) {
+    std::vector<int> left;  // places of the products still to be multiplied, in order
+    for (int j = 0; j < ng; ++j) left.push_back(j);
+    for (int next = ng; left.size() > 1;) {
         std::vector<GemmItem<double>> gi;
-        std::vector<CopyItem<double, double>> cp;
-        const int h = (k + 1) / 2;
-        for (int item = 0; item < nb; ++item) {
-            auto src = [&](int j) { return cmat(W[at], (long)item * k + j, nn); };
-            for (int j = 0; j + 1 < k; j += 2) {
-                const CMat<double> l = src(reference ? j + 1 : j), r = src(reference ? j : j + 1);
-                gi.push_back(gitem<double>(l.re, l.im, r.re, r.im, cmat(W[at ^ 1], (long)item * h + j / 2, nn), nullptr,
-                                           nullptr, nullptr, nullptr, n));
+        std::vector<int> up;
+        for (size_t j = 0; j + 1 < left.size(); j += 2, ++next) {
+            const int lo = left[j], hi = left[j + 1];
+            for (int item = 0; item < nb; ++item) {
+                const CMat<double> l = mW(item, reference ? hi : lo), r = mW(item, reference ? lo : hi);
+                gi.push_back(gitem<double>(l.re, l.im, r.re, r.im, mW(item, next), nullptr, nullptr, nullptr, nullptr, n));
             }
-            if (k % 2) cp.push_back({src(k - 1).re, cmat(W[at ^ 1], (long)item * h + h - 1, nn).re, 2 * nn});
+            up.push_back(next);
         }
-        b.add(K::GEMM64_CC, gi, n, n);
-        b.add(K::COPY64, cp, (int)(2 * nn));
+        if (left.size() % 2) up.push_back(left.back());
+        b.add(reference ? K::GEMM64_CC4 : K::GEMM64_CC, gi, n, n);
+        left = std::move(up);
     }
     std::vector<LuItem> lu;
     double* luw = b.d64(nb * lu_work_doubles(n));
     for (int item = 0; item < nb; ++item) {
-        const CMat<double> m = cmat(W[at], item, nn);
+        const CMat<double> m = mW(item, left[0]);
         lu.push_back({m.re, m.im, piv + (long)item * n, op->logdet + 2 * item, luw + item * lu_work_doubles(n), n, n});
     }
     b.add(K::LU, lu, n, 0, 1);
@@ -2109,8 +2111,10 @@ void Plan::logdetM(const double* phi, int nt, int batch, int mode, int group, in
 // reference's.  Times in MFMA cycles of a SIMD: a slice takes its tiles' products (32 n each) and about 900
 // cycles of latency (0.6 of both in FP32); a product of two groups takes its 64 x 64 tiles in rounds over
 // the CUs, 200 n each, and about 10000 to start; the force has 2 ng - 2 of those in sequence and one of all
-// K_j.  One field, one group -> this choice, in ms (a launch per slice where the strips are not used):
+// K_j, the log det one per level of its pairs.  One field, one group -> this choice, in ms (a launch per
+// slice where the strips are not used):
 //   FP64 force    n = 288, Nt 97: 5.65 -> 1.85 (3.33)   n = 384: 7.93 -> 3.00 (5.57)   n = 512: 13.5 -> 5.49 (7.69)
+//   FP64 log det  n = 288, Nt 97: 2.82 -> 1.05 (2.06)   n = 384: 4.23 -> 1.72 (3.32)   n = 512: 7.04 -> 2.99 (4.41)
 //   mixed force   n = 288, Nt 32: 1.97 -> 1.23 (2.01)   n = 384: 2.85 -> 1.85 (2.75)   n = 512: 4.70 -> 3.00 (3.67)
 // and with four fields of 32 slices one group at n = 384 (FP64 3.43; four groups 3.72) and 512.
 int Plan::chain_groups(int nt, int nb, int least, ChainUse what) {
@@ -2124,8 +2128,11 @@ int Plan::chain_groups(int nt, int nb, int least, ChainUse what) {
     for (int ng = least; ng <= std::max(least, nt / 4); ++ng) {
         const int sh = chain_shape<double>(n, nb * ng, CHAIN_CUS), len = (nt + ng - 1) / ng;
         const double slice = chain_cost(CHAIN_SHAPES[sh], tiles, nb * ng, CHAIN_CUS) * 32.0 * n * 1.15 + 900.0;
-        double c = (what == MIXED ? 1.6 : 2.0) * len * slice;
-        if (ng > 1) c += (2 * ng - 2) * product(nb) + product((long)nb * (ng - 1));
+        double c = (what == LOGDET ? 1.0 : what == MIXED ? 1.6 : 2.0) * len * slice;
+        if (what == LOGDET)
+            for (int k = ng; k > 1; k = (k + 1) / 2) c += product((long)nb * (k / 2));
+        else if (ng > 1)
+            c += (2 * ng - 2) * product(nb) + product((long)nb * (ng - 1));
         if (ng == least || c < 0.95 * cost) {
             cost = c;
             best = ng;

@@ -230,7 +230,7 @@ private:
     bool recomputes(int g) const {
         return recompute_ > 0 && recompute_ < g && g % recompute_ == 0 && nx_ % 32 == 0;
     }
-    enum ChainUse { PLAIN, MIXED };  // force in FP64, force with FP32 right chains
+    enum ChainUse { PLAIN, MIXED, LOGDET };  // force in FP64, force with FP32 right chains, log det
     std::map<std::tuple<int, int, int, int>, int> groups_;  // chain_groups' answers
     int chain_groups(int nt, int nb, int least, ChainUse what);
     template <typename OF>
