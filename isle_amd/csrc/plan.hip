@@ -1686,6 +1686,21 @@ void add_tree_logdet(Builder& b, int n, int ng, int nb, PF P, double* logdet) {
 }
 }  // namespace
 
+// Whether a slice of so many FP64 chains takes less on the strips than as a launch of its own, which splits
+// it over more workgroups.  In us: the strips as in chain_groups (at 2.4 GHz), a launch 6 + n / 100 and its
+// 4 n^3 flops at 45 TFLOP/s.  For the stable forms, whose groups are the caller's: 4 chains (one field, two groups)
+// per slice on strips / as launches: n = 192 10.7 / 12.2, 224 15.3 / 13.4, 288 26.8 / 21.8, 416 52.6 / 38.2; 6 chains
+// n = 288 27.4 / 23.5, 384 38.7 / 42.5; 12 chains n = 384 76 / 72, 416 106 / 90, 512 130 / 141 (two rounds of
+// workgroups on 256 CUs).  FP32 right chains are faster on the strips wherever that was timed.
+bool Plan::strips_pay(int chains) const {
+    const int n = nx_;
+    if (n <= CHAIN_MAX_RES) return true;
+    const int sh = chain_shape<double>(n, chains, CHAIN_CUS);
+    const double strip =
+        (chain_cost(CHAIN_SHAPES[sh], chain_tiles(n), chains, CHAIN_CUS) * 32.0 * n * 1.15 + 900.0) / 2400.0;
+    return strip <= 6.0 + 0.01 * n + chains * 4.0 * n * (double)n * n / 45e6;
+}
+
 // Stable log det M: FP64 group products (as in the grouped form), then the structured
 // factorisation of their block-cyclic matrix; per-step log-determinants are summed on the host.
 OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spin) {
@@ -1705,7 +1720,7 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
     const long nn = (long)n * n;
     const int nb = batch * nspecies;
     double* ph = b.d64((size_t)nb * 2 * nt * n);
-    const bool chains = chain_fits(n);
+    const bool chains = chain_fits(n) && strips_pay(nb * ng);
     double* Wg = b.d64((size_t)nb * ng * (chains ? 1 : 2) * 2 * nn);  // P_j, or two products in turn
     const bool tree = tree_logdet(n, ng, nb);
     op->slots = tree ? ng : ng - 1;  // log dets per item
@@ -1760,12 +1775,14 @@ OpCache& Plan::get_logdet_stable(int nt, int batch, int g, int nspecies, int spi
 // (ng-1, 0, 1, ..., ng-2) so that every step works on a prefix of the columns; then the FP64
 // right chains Rt_tau = A_s (D_tau Rt_{tau-1}) from Rt_{s_j - 1} = K_j^T and
 // f[tau] = diag(Suf_{tau+1} R_tau) as in the other forms.
-OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin, bool right32) {
+OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin, bool right32, int items) {
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
     if (right32 && nt / g < 2) throw std::invalid_argument("FP32 right chains of the stable force need two groups or more");
     // a single group is the plain form: nothing to eliminate
     if (nt == g && chain_fits(nx_)) return get_force_chains(nt, batch, nt, nspecies, spin, false, 0);
-    auto key = std::make_tuple(right32 ? 6 : 4, nt, batch, g, nspecies, spin);
+    const bool chains =
+        chain_fits(nx_) && (right32 || strips_pay((items > 0 ? items : batch * nspecies) * (nt / g)));
+    auto key = std::make_tuple(right32 ? 6 : 4, nt, batch, g, nspecies, spin + 2 * chains);
     auto found = cache_.find(key);
     if (found != cache_.end()) return *found->second;
     auto op = std::make_unique<OpCache>();
@@ -1782,7 +1799,6 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
     double* ph = b.d64((size_t)nb * 2 * nt * n);
     float* ph32 = right32 ? b.d32((size_t)nb * 2 * nt * n) : nullptr;
     double* Suf = b.d64((size_t)nb * nt * 2 * nn + 32 * (size_t)n);
-    const bool chains = chain_fits(n);
     double* Rt = right32 || chains ? nullptr : b.d64((size_t)nb * nt * 2 * nn);
     float* Rt32 = right32 && !chains ? b.d32((size_t)nb * ng * 2 * 2 * nn) : nullptr;  // last two products per group
     double* Kt = right32 || chains ? nullptr : b.d64((size_t)nb * ng * 2 * nn);
@@ -2149,7 +2165,7 @@ OpCache& Plan::get_force(int mode, int nt, int batch, int group, int nspecies, i
     }
     return mode == 0   ? get_force_plain(nt, batch, nspecies, spin)
            : mode == 1 ? get_force_mixed(nt, batch, group, nspecies, spin)
-                       : get_force_stable(nt, batch, group, nspecies, spin, mode == 3);
+                       : get_force_stable(nt, batch, group, nspecies, spin, mode == 3, items);
 }
 
 void Plan::force_parts(const double* phi, int nt, int batch, int mode, int group, int nspecies, int spin,

@@ -233,6 +233,7 @@ private:
     enum ChainUse { PLAIN, MIXED, LOGDET };  // force in FP64, force with FP32 right chains, log det
     std::map<std::tuple<int, int, int, int>, int> groups_;  // chain_groups' answers
     int chain_groups(int nt, int nb, int least, ChainUse what);
+    bool strips_pay(int chains) const;
     template <typename OF>
     void add_suffix(Builder& b, const std::vector<int>& at, int nb, int nspecies, const double* ph, OF out, long step,
                     int all);
@@ -243,7 +244,7 @@ private:
     OpCache& get_logdet_plain(int nt, int batch, int nspecies, int spin);
     OpCache& get_logdet_chains(int nt, int batch, int g, int nspecies, int spin, bool reference);
     OpCache& get_logdet_grouped(int nt, int batch, int group, int nspecies, int spin);
-    OpCache& get_force_stable(int nt, int batch, int group, int nspecies, int spin, bool right32 = false);
+    OpCache& get_force_stable(int nt, int batch, int group, int nspecies, int spin, bool right32 = false, int items = 0);
     OpCache& get_logdet_stable(int nt, int batch, int group, int nspecies, int spin);
     struct QBlocks {
         double *p, *tplus, *tminus;  // P; T+(t), T-(t) (re plane, im plane, nt of each)
