@@ -1572,12 +1572,16 @@ Cyclic add_cyclic_factor(Builder& b, int n, int ng, int nb, PF P, double* logdet
 //
 // A merge of two products eliminates 2 n full rows, half again the work of a leaf, so the tree pays while
 // the sequence of panels is the longer part: its time goes like n per factorisation, the work like nb n^3.
-// Sequence -> tree in ms, n = 288: ng = 16: nb = 2 13.1 -> 5.0, 32 26.3 -> 22.1, 48 33.7 -> 32.0, 64 41.8 -> 42.0,
-// 96 60.2 -> 62.0; nb = 32: ng = 8 12.5 -> 11.3, 6 9.15 -> 9.03, 4 5.77 -> 5.90; nb = 2: ng = 4 3.09 -> 2.56, 3
-// 2.30 -> 2.44; n = 128, ng = 8: nb = 96 4.72 -> 4.16, 192 7.39 -> 7.60; n = 384: nb = 8, ng = 16 24.4 -> 15.2,
-// nb = 64, ng = 32 196 -> 190.  n <= 384: the 2 n candidate rows of a merge then fit the registers of a workgroup.
+// Sequence -> tree in ms, n = 288: ng = 4: nb = 8 3.18 -> 2.76, 16 3.65 -> 3.38, 24 4.02 -> 3.96, 32 4.45 -> 4.64;
+// ng = 8: nb = 32 10.2 -> 9.1, 40 11.4 -> 10.9, 48 12.6 -> 12.7; ng = 12: nb = 48 19.8 -> 19.5, 56 21.5 -> 22.2;
+// ng = 16: nb = 2 (8 slices a group) 13.1 -> 5.0, 48 26.8 -> 25.5, 56 29.2 -> 29.4, 64 32.9 -> 33.2; ng = 32: nb = 96
+// 115 -> 103.  n = 128: ng = 8: nb = 96 4.01 -> 3.54, 160 5.28 -> 5.47; ng = 4: nb = 64 1.52 -> 1.42, 96 1.81 -> 1.83.
+// n = 384: ng = 8: nb = 16 12.5 -> 10.7; ng = 16: nb = 32 37.3 -> 37.4.  ng = 3, n = 288, nb = 2: 2.30 -> 2.44.
+// So the line is drawn at four matrices of order 288 per group (TREE_WORK), and matrices on it take the tree for
+// fewer than 16 groups.  n <= 384: the 2 n candidate rows of a merge then fit the registers of a workgroup.
+constexpr long TREE_WORK = 4L * 288 * 288;
 inline bool tree_logdet(int n, int ng, int nb) {
-    return ng >= 4 && 2 * n <= LU_MID_N && (double)nb * n * n < 331776.0 * ng;
+    return ng >= 4 && 2 * n <= LU_MID_N && (long)nb * n * n - TREE_WORK * ng < (ng < 16 ? 1 : 0);
 }
 template <typename PF>
 void add_tree_logdet(Builder& b, int n, int ng, int nb, PF P, double* logdet) {
