@@ -228,20 +228,11 @@ void add_trsm(Builder& b, int mode, int n, int w, const std::vector<TrsmMat>& ma
         }
     }
 }
-// Whether the inverses of nb factorised matrices take blocked triangular solves on GEMMs (four launches per pair
-// of panels, on all CUs) rather than lu_solve_kernel (one launch, a workgroup per 16 columns, each with the whole
-// chain of panels).  Mixed force of 16 or 32 slices, us with lu_solve_kernel / blocked: n = 64: nb = 64 257 / 271, 256
-// 516 / 520; n = 128: nb = 8 414 / 433, 64 573 / 619, 256 1566 / 1548; n = 192: nb = 32 991 / 1023, 64 1399 / 1385;
-// n = 224: nb = 16 926 / 969, 32 1479 / 1399; n = 288: nb = 8 1398 / 1392, 12 1445 / 1504, 16 2056 / 1855 (a second
-// round of workgroups); n = 320: nb = 2 1254 / 1231, 12 1652 / 1698, 16 2544 / 2287; n = 352: nb = 2 1419 / 1364, 8
-// 1848 / 1841; n = 448: nb = 2 2131 / 2010, 8 2808 / 2769.
-inline bool trsm_inverse(int n, int nb) {
-    return n % LU_NB == 0 && (n > 320 || (double)nb * n * n * n > 3.4e8);
-}
 // Top level of the grouped force in FP64, from the group products P(item, j):
 //   GL_{ng-1} = I, GL_j = P_{j+1} GL_{j+1};  Mid = (1 + P_0 GL_0)^{-1}
 //   RR_0 = Mid, RR_j = RR_{j-1} P_{j-1};     K_j = GL_j RR_j
-// trsm: the inverse by blocked triangular solves on GEMMs (n % 32 == 0), else by lu_solve_kernel.  keep: P_0 is read again afterwards;
+// trsm: the inverse by blocked triangular solves on GEMMs (n % 32 == 0; many matrices), else by
+// lu_solve_kernel (few: one launch instead of four per pair of panels).  keep: P_0 is read again afterwards;
 // with a single group it is otherwise factorised in place.
 struct TopLevel {
     double *KK, *RR;
@@ -1204,7 +1195,7 @@ OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin
     b.add(K::PHASE, phs);
     add_suffix(b, at, nb, nspecies, ph, [&](int item, int j) { return mS(item, at[j + 1] - 1).re; }, -2 * nn, 1);
     const TopLevel tl = add_top_level(b, n, ng, nb, [&](int item, int j) { return mS(item, at[j]); },
-                                      trsm_inverse(n, nb), false);
+                                      n % LU_NB == 0 && nb > 4, false);
     add_right(b, *op, at, nb, nspecies, ph, ph32, Suf, [&](int item, int j) { return ChainK{tl.k(item, j), nn, n, 1.0}; });
     b.finish();
     tune(*op);
