@@ -1164,10 +1164,12 @@ OpCache& Plan::get_force_mixed(int nt, int batch, int g, int nspecies, int spin)
 // The grouped force on the strip kernels (chain.hpp): every group's suffix chain in one launch,
 // the top level, every group's right chain with the diagonal fused in one launch.  right32: the
 // mixed form (FP32 right chains); else FP64 throughout.  g: most slices of a group (chain_groups may
-// take shorter ones); items: (field, species) pairs that share the launches, 0 for this batch's alone.
-OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin, bool right32, int items) {
+// take shorter ones).  shared: the batch is one of several whose operations run merged; the mixed form then keeps
+// to the given groups, which line up over the batches (fields of 18, 36 and 72 slices at n = 288, three of each:
+// 13% slower with groups of their own).
+OpCache& Plan::get_force_chains(int nt, int batch, int g, int nspecies, int spin, bool right32, bool shared) {
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
-    const int ng = chain_groups(nt, items > 0 ? items : batch * nspecies, nt / g, right32 ? MIXED : PLAIN);
+    const int ng = right32 && shared ? nt / g : chain_groups(nt, batch * nspecies, nt / g, right32 ? MIXED : PLAIN);
     auto key = std::make_tuple(right32 ? 1 : 0, nt, batch, g, nspecies, spin + 2 * ng);
     auto found = cache_.find(key);
     if (found != cache_.end()) return *found->second;
@@ -1783,7 +1785,7 @@ OpCache& Plan::get_force_stable(int nt, int batch, int g, int nspecies, int spin
     if (g <= 0 || nt % g != 0) throw std::invalid_argument("group size must divide nt");
     if (right32 && nt / g < 2) throw std::invalid_argument("FP32 right chains of the stable force need two groups or more");
     // a single group is the plain form: nothing to eliminate
-    if (nt == g && chain_fits(nx_)) return get_force_chains(nt, batch, nt, nspecies, spin, false, 0);
+    if (nt == g && chain_fits(nx_)) return get_force_chains(nt, batch, nt, nspecies, spin, false, items > 0);
     const bool chains =
         chain_fits(nx_) && (right32 || strips_pay((items > 0 ? items : batch * nspecies) * (nt / g)));
     auto key = std::make_tuple(right32 ? 6 : 4, nt, batch, g, nspecies, spin + 2 * chains);
@@ -2124,48 +2126,67 @@ void Plan::logdetM(const double* phi, int nt, int batch, int mode, int group, in
 }
 
 // Groups of the strip chains of nb (field, species) items, at least `least` of them: that many, or, for
-// n > CHAIN_MAX_RES, the number with the shortest time where few items leave the GPU idle.  The result is
-// as accurate either way (ten fields each, n = 144 .. 384, Nt 31 .. 97: errors against 64 bits 0.8 to 1.3 of
-// one chain's), but rounded differently, so an item's last bits depend on nb.  Up to CHAIN_MAX_RES a slice
-// takes 3 us and grouping gave 4% of a gradient at n = 72, not worth an order of products other than the
-// reference's.  Times in MFMA cycles of a SIMD: a slice takes its tiles' products (32 n each) and about 900
-// cycles of latency (0.6 of both in FP32); a product of two groups takes its 64 x 64 tiles in rounds over
-// the CUs, 200 n each, and about 10000 to start; the force has 2 ng - 2 of those in sequence and one of all
-// K_j, the log det one per level of its pairs.  One field, one group -> this choice, in ms (a launch per
-// slice where the strips are not used):
+// n > CHAIN_MAX_RES, more where few items leave the GPU idle: for the FP64 force the divisor of nt with the shortest
+// time, and any number that saves 10% against that (or against `least`), so that results move in their last bits
+// only for a gain.  They are as accurate either way (50 to 80 fields each, n = 180 .. 512: errors of the force against
+// 64 bits 0.95 to 1.1 of those of one chain, +- 0.04 to 0.09), but an item's last bits depend on nb.  Up to
+// CHAIN_MAX_RES a slice takes 3 us, and grouping gave 4% of a gradient at n = 72: not worth an order of products other
+// than the reference's.
+// Times in MFMA cycles of a SIMD: a slice takes its tiles' products (32 n each) and about 900 cycles of latency (0.6
+// of both in FP32).  A product of two groups takes its 64 x 64 tiles in rounds over the CUs, 200 n each, and 10000
+// cycles; between divisors, whose group numbers lie further apart, 7000 cycles and a share of n^3 decide.  The force
+// has 2 ng - 2 products in sequence and one of all K_j, the log det (pairwise) one per level.  Over orders 144 to 512,
+// 16 to 97 slices and 1 to 8 fields the choice is 0.8% above the best of 1 to 16 groups on average (force; 0.4% log det,
+// 0.1% mixed), 9% at worst.  One field, one group -> this choice, in ms (a launch per slice where the strips are not
+// used):
 //   FP64 force    n = 288, Nt 97: 5.65 -> 1.85 (3.33)   n = 384: 7.93 -> 3.00 (5.57)   n = 512: 13.5 -> 5.49 (7.69)
 //   FP64 log det  n = 288, Nt 97: 2.82 -> 1.05 (2.06)   n = 384: 4.23 -> 1.72 (3.32)   n = 512: 7.04 -> 2.99 (4.41)
 //   mixed force   n = 288, Nt 32: 1.97 -> 1.23 (2.01)   n = 384: 2.85 -> 1.85 (2.75)   n = 512: 4.70 -> 3.00 (3.67)
-// and with four fields of 32 slices one group at n = 384 (FP64 3.43; four groups 3.72) and 512.
 int Plan::chain_groups(int nt, int nb, int least, ChainUse what) {
     const int n = nx_, tiles = chain_tiles(n);
     if (n <= CHAIN_MAX_RES) return least;
     int& best = groups_[std::make_tuple(nt, nb, least, (int)what)];
     if (best > 0) return best;
+    const double n3 = (double)n * n * n;
     const long t64 = (long)cdiv(n, 64) * cdiv(n, 64);
     auto product = [&](long items) { return 10000.0 + 200.0 * n * ((items * t64 + CHAIN_CUS - 1) / CHAIN_CUS); };
-    double cost = 0;
-    for (int ng = least; ng <= std::max(least, nt / 4); ++ng) {
+    auto slices = [&](int ng) {  // of a group's chain
         const int sh = chain_shape<double>(n, nb * ng, CHAIN_CUS), len = (nt + ng - 1) / ng;
-        const double slice = chain_cost(CHAIN_SHAPES[sh], tiles, nb * ng, CHAIN_CUS) * 32.0 * n * 1.15 + 900.0;
-        double c = (what == LOGDET ? 1.0 : what == MIXED ? 1.6 : 2.0) * len * slice;
+        return len * (chain_cost(CHAIN_SHAPES[sh], tiles, nb * ng, CHAIN_CUS) * 32.0 * n * 1.15 + 900.0);
+    };
+    auto cost = [&](int ng) {
+        double c = (what == LOGDET ? 1.0 : what == MIXED ? 1.6 : 2.0) * slices(ng);
         if (what == LOGDET)
             for (int k = ng; k > 1; k = (k + 1) / 2) c += product((long)nb * (k / 2));
         else if (ng > 1)
             c += (2 * ng - 2) * product(nb) + product((long)nb * (ng - 1));
-        if (ng == least || c < 0.95 * cost) {
-            cost = c;
+        return c;
+    };
+    best = least;
+    double c0 = 0;
+    for (int ng = least; what == PLAIN && ng <= std::max(least, nt / 4); ++ng) {
+        if (nt % ng != 0) continue;
+        const double c = 2.0 * slices(ng) + (ng > 1 ? (2 * ng - 1) * (7000.0 + 0.0016 * n3 * std::max(1.0, nb / 8.0)) : 0.0);
+        if (ng == least || c < 0.95 * c0) {
             best = ng;
+            c0 = c;
         }
     }
+    const int even = best;
+    c0 = cost(even);
+    for (int ng = least + 1; ng <= nt / 4; ++ng)
+        if (cost(ng) < (best == even ? 0.9 : 0.95) * c0) {
+            best = ng;
+            c0 = cost(ng);
+        }
     return best;
 }
 
 OpCache& Plan::get_force(int mode, int nt, int batch, int group, int nspecies, int spin, int items) {
     if (nt < 2) throw std::invalid_argument("nt < 2 in HubbardFermiAction algorithm DIRECT_SINGLE not supported");
     if (chain_fits(nx_)) {
-        if (mode == 0) return get_force_chains(nt, batch, nt, nspecies, spin, false, items);
-        if (mode == 1 && !recomputes(group)) return get_force_chains(nt, batch, group, nspecies, spin, true, items);
+        if (mode == 0) return get_force_chains(nt, batch, nt, nspecies, spin, false, items > 0);
+        if (mode == 1 && !recomputes(group)) return get_force_chains(nt, batch, group, nspecies, spin, true, items > 0);
     }
     return mode == 0   ? get_force_plain(nt, batch, nspecies, spin)
            : mode == 1 ? get_force_mixed(nt, batch, group, nspecies, spin)

@@ -240,7 +240,7 @@ private:
     template <typename KF>
     void add_right(Builder& b, OpCache& op, const std::vector<int>& at, int nb, int nspecies, const double* ph,
                    const float* ph32, const double* Suf, KF kf);
-    OpCache& get_force_chains(int nt, int batch, int group, int nspecies, int spin, bool right32, int items);
+    OpCache& get_force_chains(int nt, int batch, int group, int nspecies, int spin, bool right32, bool shared);
     OpCache& get_logdet_plain(int nt, int batch, int nspecies, int spin);
     OpCache& get_logdet_chains(int nt, int batch, int g, int nspecies, int spin, bool reference);
     OpCache& get_logdet_grouped(int nt, int batch, int group, int nspecies, int spin);
