@@ -692,7 +692,8 @@ def main():
         "speedup_vs_plain_fp64": (traj_per_s / plain) if plain else None,
         "plain_fp64_batched_traj_per_s": plain_batched,
         "speedup_vs_plain_fp64_batched": (traj_per_s / plain_batched) if plain_batched else None,
-        "plain_note": f"plain FP64 = the reference's algorithm in FP64 on the same kernels; single chain and "
+        "plain_note": f"plain FP64 = every product in FP64 on the same kernels (the reference's factors of the force; "
+                      f"its chain of slices cut into groups where few chains leave the GPU idle); single chain and "
                       f"{B} batched chains, {args.plain_steps} timed trajectories each after one warm-up",
         "force_rel_err": force_err, "force_rel_err_max": force_err_max,
         "force_rel_err_note": "max over the chains' thermalised fields of |F_mixed - F_fp64|_2 / |F_fp64|_2 "

@@ -231,9 +231,14 @@ void add_trsm(Builder& b, int mode, int n, int w, const std::vector<TrsmMat>& ma
 // Top level of the grouped force in FP64, from the group products P(item, j):
 //   GL_{ng-1} = I, GL_j = P_{j+1} GL_{j+1};  Mid = (1 + P_0 GL_0)^{-1}
 //   RR_0 = Mid, RR_j = RR_{j-1} P_{j-1};     K_j = GL_j RR_j
-// trsm: the inverse by blocked triangular solves on GEMMs (n % 32 == 0; many matrices), else by
-// lu_solve_kernel (few: one launch instead of four per pair of panels).  keep: P_0 is read again afterwards;
-// with a single group it is otherwise factorised in place.
+// trsm: the inverse by blocked triangular solves on GEMMs (n % 32 == 0), else by lu_solve_kernel (one launch instead
+// of four per pair of panels).  get_force_chains draws the line at four matrices.  Mixed force of 16 or 32 slices, us
+// with lu_solve_kernel / blocked: n = 64: nb = 2 233 / 242, 64 257 / 271, 256 516 / 520; n = 128: 8 414 / 433, 64 573 /
+// 619, 256 1566 / 1548; n = 192: 32 991 / 1023, 64 1399 / 1385; n = 224: 16 926 / 969, 32 1479 / 1399; n = 288: 2 1090 /
+// 1088, 8 1398 / 1392, 12 1445 / 1504, 16 2056 / 1855, 32 3061 / 2723; n = 352: 2 1419 / 1364, 8 1848 / 1841; n = 448:
+// 2 2131 / 2010.  A line that follows these (n > 320, or nb n^3 > 3.4e8) saves up to 8% of small batches, but moves
+// the last bits of FP64 forces on either side of it, visibly where det M is near a zero.
+// keep: P_0 is read again afterwards; with a single group it is otherwise factorised in place.
 struct TopLevel {
     double *KK, *RR;
     int ng;
